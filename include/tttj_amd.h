@@ -169,8 +169,8 @@ int tt_layernorm_fwd(const void* x, const void* gamma, const void* beta, const u
                      void* y, int rows, int d, float eps, void* stream);
 
 /* Y[M,N] = X[M,K] W[N,K]^T + b with one of the TT_EPI_* epilogues; fp16 in/out, fp32 accumulate
- * on MFMA when K % 64 == 0 and N % 64 == 0, else (N, K multiples of 8, e.g. d_model 32) on a
- * small vector-ALU kernel with the same epilogues.  M * K may exceed 2^31; N * K may not.  For
+ * on MFMA; N and K multiples of 8 (multiples of 64 run on the tiles tt_gemm_tile_override names,
+ * others on ragged forms of three of them).  M * K may exceed 2^31; N * K may not.  For
  * TT_EPI_QKV, N == 3*D with D = heads*head_dim and M == batch*seq.  Replaces _linear_tile with EPILOGUE 0-3 (kernels/fused_megakernel.py:447-541),
  * linear_gelu (kernels/case13_linear.py:149-176), the packed-QKV F.linear
  * (kernels/layerwise_hybrid.py:188-192) and _head_major_qkv_kernel (case13_linear.py:114-146). */

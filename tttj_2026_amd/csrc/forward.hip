@@ -99,9 +99,10 @@ static Workspace carve(char* base, int64_t B, int64_t S, int64_t D, int64_t F) {
 }
 
 // Whether the layer-wise plan folds LN2 (and LN1 of layers >= 1) into the next projection: only
-// where both QKV and ffn_in run on the narrow / small kernels (few tokens).
+// where both QKV and ffn_in run on the narrow kernels (few tokens), whose statistics slots are 32
+// columns wide.
 static bool folds_layernorm(bool fused_ln, int64_t T, int64_t D, int64_t F) {
-  return !fused_ln && linear_is_narrow((int)T, (int)(3 * D), (int)D, TT_EPI_QKV) &&
+  return !fused_ln && D % 32 == 0 && linear_is_narrow((int)T, (int)(3 * D), (int)D, TT_EPI_QKV) &&
          linear_is_narrow((int)T, (int)F, (int)D, TT_EPI_BIAS_GELU);
 }
 
@@ -444,7 +445,7 @@ int transformer_fwd(const void* weights, const void* x, const uint8_t* mask, voi
   const int ldp = D / 4;     // float2 slots per row of ws.part (the narrowest producer: 4 columns)
   int part_slots = 0;        // slots per row the last producer wrote
   // The fold pays only where launches dominate: for few tokens, whose QKV / ffn_in GEMMs run on
-  // the narrow / small kernels (the statistics loads overlap their K loop).  On the MFMA tiles of
+  // the narrow kernels (the statistics loads overlap their K loop).  On the MFMA tiles of
   // larger shapes the epilogue work it adds is exposed and costs more than the LayerNorm launch
   // it removes (measured on MI355X: C5 +3.9%, C4 +5.5%), so LN1 / LN2 stay standalone there.
   const bool fold = folds_layernorm(fused_ln, T, D, F);

@@ -16,8 +16,8 @@ struct EpiArgs {
   // TT_EPI_QKV: factor on the Q columns before their fp16 rounding.  The forward passes
   // hd^-1/2 log2(e), the form its attention launches read Q in (AttnArgs::q_prescaled).
   float q_scale = 1.f;
-  // LayerNorm folded into this projection (TT_EPI_QKV / TT_EPI_BIAS_GELU, on the narrow and
-  // small kernels): X is the raw residual stream, W = W diag(gamma), and the epilogue computes
+  // LayerNorm folded into this projection (TT_EPI_QKV / TT_EPI_BIAS_GELU, on the narrow
+  // kernels): X is the raw residual stream, W = W diag(gamma), and the epilogue computes
   // rstd (acc - mean c) + b' instead of acc + bias.  The row statistics come from ln_slots
   // partial (mean, M2) slots per row (row stride ln_stride float2), each over K / ln_slots
   // columns.
@@ -48,10 +48,14 @@ int launch_layernorm_rows(const half* x, const half* gamma, const half* beta, co
 
 int launch_linear(const half* x, const half* w, int m, int n, int k, const EpiArgs& ep,
                   hipStream_t stream);
+// Tiles of the GEMM kernels for ragged widths (gemm_ragged.hip).
+enum class RaggedTile { kNarrow, k64x64, k128x128 };
+int run_ragged(RaggedTile tile, const half* x, const half* w, int m, int n, int k, const EpiArgs& ep,
+               hipStream_t stream);
 // Columns per partial-statistics slot the GEMM launch_linear would run for this shape writes
-// (the column range of one wave, or of one thread group on the narrow and small kernels).
+// (the column range of one wave, or of one thread group on the narrow kernels).
 int linear_stats_width(int m, int n, int k, int mode);
-// Whether launch_linear runs this shape on the narrow (32 x 32) or small (vector-ALU) kernel.
+// Whether launch_linear runs this shape on the narrow (32 x 32) kernels.
 bool linear_is_narrow(int m, int n, int k, int mode);
 
 // Derived segments 12-17 of the packed weights (lnfold.hip).
