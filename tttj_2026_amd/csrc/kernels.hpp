@@ -97,7 +97,7 @@ struct AttnArgs;
 // head_dim 256: the MFMA flash block with accumulators in AGPRs (attention_wide.hip).
 int launch_attention_wide(const AttnArgs& args, const int32_t* info, int head_dim, int causal,
                           hipStream_t stream);
-// head_dim 8 / 16: one lane per query, scores and P V on the vector ALUs (attention_small.hip).
+// head_dim 8 / 16: 16-wide MFMA tiles, probabilities in fp32 precision (attention_small.hip).
 int launch_attention_small(const AttnArgs& args, const int32_t* info, int head_dim, int causal,
                            hipStream_t stream);
 
