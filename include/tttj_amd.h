@@ -68,7 +68,9 @@ int tt_device_count(void);
  *   14 bqkv'[3D] fp32 = bqkv + Wqkv norm1.bias  15 W1'[F,D] = ffn_in.weight diag(norm2.weight)
  *   16 c1[F] fp32 = row sums of W1'  17 b1'[F] fp32 = ffn_in.bias + ffn_in.weight norm2.bias
  * (fp32 segments hold two fp16 slots per value), then final_norm.weight[D], final_norm.bias[D]
- * after the last layer.  Writes the TT_LAYER_SEGMENTS per-layer segment offsets (elements,
+ * after the last layer, and behind them, for d_model <= 192 and ffn_dim <= 1024 (both multiples of
+ * 32), a region that only tt_pack_derived and the forward use (the layers' weights in matrix
+ * fragment order), counted in the total.  Writes the TT_LAYER_SEGMENTS per-layer segment offsets (elements,
  * relative to the layer start), the layer stride, the final-norm offset and the total element
  * count. */
 #define TT_LAYER_SEGMENTS 18
@@ -76,8 +78,9 @@ int tt_weight_layout(int d_model, int ffn_dim, int num_layers,
                      int64_t layer_offsets[TT_LAYER_SEGMENTS], int64_t* layer_stride,
                      int64_t* final_norm_offset, int64_t* total_elems);
 
-/* Fill segments 12-17 of every layer of a packed weight buffer from its segments 0-11 (one kernel
- * launch on `stream`; call after the base segments are written and whenever they change).  With
+/* Fill segments 12-17 of every layer of a packed weight buffer, and the region behind the final
+ * norm, from its segments 0-11 (one or two kernel launches on `stream`; call after the base
+ * segments are written and whenever they change).  With
  * LayerNorm y = (x - mean) rstd gamma + beta, LN(x) W^T + b = rstd (x W'^T - mean c) + b': the
  * layer-wise plan then multiplies the raw residual stream by W' and applies the per-row
  * statistics in the GEMM epilogue instead of launching a LayerNorm.  No counterpart in the
@@ -93,7 +96,9 @@ int tt_pack_derived(void* weights, int d_model, int ffn_dim, int num_layers, voi
                               * layer-wise.  When AUTO resolves to the megakernel
                               * (tt_resolve_plan), its workspace rules apply: zero-filled before
                               * the first call and kept for that one shape. */
-#define TT_PLAN_LAYERWISE 1  /* one launch per op: LN, GEMMs with fused epilogues, attention */
+#define TT_PLAN_LAYERWISE 1  /* one launch per op: LN, GEMMs with fused epilogues, attention; for
+                              * d_model <= 192 and ffn_dim <= 1024 (both multiples of 32) attention
+                              * and one row-chain launch per layer, as TT_PLAN_FUSED_LN then */
 #define TT_PLAN_MEGAKERNEL 2 /* one persistent launch (<= one workgroup per CU) for the stack */
 #define TT_PLAN_FUSED_LN 3   /* layer-wise with LN1 / LN2 computed inside the QKV / ffn_in GEMM
                               * tiles (five launches per layer; d_model <= 512) */

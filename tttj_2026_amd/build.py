@@ -40,6 +40,7 @@ HIPCC_FLAGS = [
 SOURCE_FLAGS = {
     "attention.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "attention_small.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "rowchain.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "megakernel.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 

@@ -36,12 +36,13 @@ static size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
 struct Layout {
   int64_t off[TT_LAYER_SEGMENTS];
-  int64_t stride, final_off, total;
+  int64_t stride, final_off, frag_off, total;
 };
 
 // Segments 12-17 are derived from 0-11 (tt_pack_derived): the QKV and ffn_in weights with the
 // LayerNorm gain folded in, W' = W diag(gamma) (fp16), their row sums c = sum_k W'[n, k] and the
-// folded biases b' = b + W beta (both fp32, two halfs per value).
+// folded biases b' = b + W beta (both fp32, two halfs per value).  After the final norm come, for narrow
+// models, the fragment-order copies of every layer's weights that the row chain reads.
 static Layout weight_layout(int64_t D, int64_t F, int64_t L) {
   const int64_t sizes[TT_LAYER_SEGMENTS] = {D, D, 3 * D * D, 3 * D, D * D, D, D, D, F * D, F, D * F,
                                             D, 3 * D * D, 6 * D, 6 * D, F * D, 2 * F, 2 * F};
@@ -53,7 +54,8 @@ static Layout weight_layout(int64_t D, int64_t F, int64_t L) {
   }
   lay.stride = o;
   lay.final_off = L * o;
-  lay.total = lay.final_off + 2 * align64(D);
+  lay.frag_off = lay.final_off + 2 * align64(D);
+  lay.total = lay.frag_off + L * chain_fragment_halfs(D, F);
   return lay;
 }
 
@@ -106,6 +108,8 @@ static bool folds_layernorm(bool fused_ln, int64_t T, int64_t D, int64_t F) {
          linear_is_narrow((int)T, (int)F, (int)D, TT_EPI_BIAS_GELU);
 }
 
+static bool chains_rows(bool masked, int64_t B, int64_t S, int64_t D, int64_t H, int64_t F);
+
 // Whether a masked layer-wise forward packs the valid tokens (varlen.hip): when the LayerNorms
 // are not fused or folded and all four projections run on the MFMA tiles (the packed row count
 // is read on the device by those kernels), and the Q / V^T planes stay below 2^31 elements.
@@ -114,12 +118,26 @@ static bool g_packing_off = false;  // test hook (tt_forward_packing_override)
 static bool packs_rows(bool fused_ln, bool fold, int64_t B, int64_t S, int64_t D, int64_t H,
                        int64_t F) {
   const int64_t T = B * S, Sp = (S + 63) / 64 * 64;
-  if (g_packing_off || fused_ln || fold || T * D >= (1LL << 31) || B * D * Sp >= (1LL << 31))
+  if (g_packing_off || fused_ln || fold || chains_rows(true, B, S, D, H, F) || T * D >= (1LL << 31) || B * D * Sp >= (1LL << 31))
     return false;
   return !linear_is_narrow((int)T, (int)(3 * D), (int)D, TT_EPI_QKV) &&
          !linear_is_narrow((int)T, (int)D, (int)D, TT_EPI_RESID_MASKED) &&
          !linear_is_narrow((int)T, (int)F, (int)D, TT_EPI_BIAS_GELU) &&
          !linear_is_narrow((int)T, (int)D, (int)F, TT_EPI_MASKED_RESID) && H > 0;
+}
+
+// Whether the layer-wise and fused-LN plans run each layer as attention + row chain (rowchain.hip): narrow
+// models, where a 32-row block's share of the layer's weights streams from the L2 faster than five to seven
+// launches.  Measured on MI355X, whole forwards, launches per op -> row chain: D 128, F 128, 4 layers, S 128: B 1
+// 93 -> 51 us (fused-LN tiles), B 64 144 -> 67, B 10000 7576 -> 4970; D 128, F 512, 32 x 1024 tokens, 2 layers
+// 200 -> 122; D 192, F 768 the same 250 -> 203; D 160, F 640, 1600 tokens, one layer 40 -> 29.  At D 256 every block
+// streams four times the bytes of D 128 and the GEMM tiles win (4 x 128 tokens, F 1024: 60 -> 123 us; 32 x 512: 192
+// -> 252, with a first form of the kernel).
+static bool chains_rows(bool masked, int64_t B, int64_t S, int64_t D, int64_t H, int64_t F) {
+  const int64_t T = B * S, Sp = (S + 63) / 64 * 64;
+  if (chain_fragment_halfs(D, F) == 0) return false;
+  if (T * D >= (1LL << 31) || B * D * Sp >= (1LL << 31)) return false;
+  return !masked || T <= (1LL << 20);  // larger padded batches pack their rows
 }
 
 static int check_model_shape(int B, int S, int D, int H, int F, int L) {
@@ -167,8 +185,11 @@ extern "C" int tt_pack_derived(void* weights, int d_model, int ffn_dim, int num_
   TT_REQUIRE(weights != nullptr && d_model > 0 && ffn_dim > 0 && num_layers > 0,
              "pack_derived: bad arguments");
   const Layout lay = weight_layout(d_model, ffn_dim, num_layers);
-  return launch_pack_derived((half*)weights, lay.stride, lay.off, d_model, ffn_dim, num_layers,
-                             (hipStream_t)stream);
+  const int rc = launch_pack_derived((half*)weights, lay.stride, lay.off, d_model, ffn_dim, num_layers,
+                                     (hipStream_t)stream);
+  if (rc != TT_OK) return rc;
+  return launch_pack_fragments((const half*)weights, lay.stride, lay.off, (half*)weights + lay.frag_off,
+                               d_model, ffn_dim, num_layers, (hipStream_t)stream);
 }
 
 // Token count up to which the automatic plan runs the persistent megakernel (d_model >= 256).
@@ -182,7 +203,9 @@ static constexpr int kMegaMaxDModel = 512;  // the megakernel keeps a LayerNorm'
 // the latency-bound path) only for narrow models with few tokens: measured on MI355X, d_model 128
 // gains up to 2048 tokens (the reference's cases 2-4: 94 / 92 / 102 us fused against 101 / 97 /
 // 115 layer-wise) and loses from 8192 (case 1: 161 against 147 us); at d_model 256 the layer-wise
-// plan with narrow GEMM tiles is as fast or faster (C1 68 / 68 us, C2 106 against 118 us).
+// plan with narrow GEMM tiles is as fast or faster (C1 68 / 68 us, C2 106 against 118 us).  Both
+// plans take the row chain first where it applies (chains_rows), which leaves the tiles ffn_dim
+// above 1024 and explicit plans above d_model 192.
 static constexpr int64_t kFusedLnMaxTokens = 2048;
 static constexpr int kFusedLnMaxDModel = 128;
 
@@ -236,7 +259,8 @@ extern "C" int tt_stage_offsets(int batch, int seq, int d_model, int num_heads, 
   *hidden = (int64_t)w.off_hbuf;
   // the context buffer is overwritten by the LN2 output unless LN2 is fused or folded
   const bool fused_ln = plan == TT_PLAN_FUSED_LN;
-  *ctx = (fused_ln || folds_layernorm(fused_ln, (int64_t)batch * seq, d_model, ffn_dim))
+  *ctx = (fused_ln || folds_layernorm(fused_ln, (int64_t)batch * seq, d_model, ffn_dim) ||
+          chains_rows(true, batch, seq, d_model, num_heads, ffn_dim))
              ? (int64_t)w.off_xn
              : -1;
   return TT_OK;
@@ -385,6 +409,53 @@ static int forward_packed(const half* wts, const Layout& lay, const half* x, con
                                ws.slot, nullptr, nullptr, y, T, D, 1e-5f, stream);
 }
 
+// Layer-wise forward of a narrow model: LN1 + QKV of layer 0, then per layer the attention and the row
+// chain up to the next layer's QKV projection or the final norm (2 L + 1 launches, one more with a mask).
+static int forward_chained(const half* wts, const Layout& lay, const half* x, const uint8_t* mask, half* y,
+                           const Workspace& ws, const int32_t* info, int B, int S, int D, int H, int F,
+                           int L, int causal, hipStream_t stream) {
+  const int hd = D / H;
+  const size_t plane = (size_t)B * S * D;
+  ChainArgs a{};
+  for (int i = 0; i < TT_LAYER_SEGMENTS; ++i) a.off[i] = lay.off[i];
+  a.fin_g = wts + lay.final_off;
+  a.fin_b = a.fin_g + align64(D);
+  a.ctx = ws.xn;
+  a.xa = ws.xa;
+  a.q = ws.qkv;
+  a.valid = mask;
+  a.T = B * S;
+  a.S = S;
+  a.H = H;
+  a.hd = hd;
+  for (a.hd_log2 = 0; (1 << a.hd_log2) < hd; ++a.hd_log2) {
+  }
+  a.F = F;
+  a.ldv = (S + 63) / 64 * 64;
+  a.q_scale = attention_q_scale(hd);
+  a.x = x;
+  a.wn = wts;
+  const int64_t per = chain_fragment_halfs(D, F);
+  a.fw = a.fwn = wts + lay.frag_off;
+  int rc = launch_rowchain(a, D, false, stream);
+  for (int l = 0; rc == TT_OK && l < L; ++l) {
+    if ((rc = launch_attention(ws.qkv, ws.qkv + plane, ws.qkv + 2 * plane, mask, info, ws.xn, B, S, H, hd,
+                               causal, stream, true)) != TT_OK)
+      break;
+    a.w = wts + (size_t)l * lay.stride;
+    a.wn = a.w + lay.stride;  // not read after the last layer
+    a.fw = wts + lay.frag_off + l * per;
+    a.fwn = a.fw + per;
+    a.x = l == 0 ? x : ws.xa;
+    if (l + 1 == L) {
+      a.y = y;
+      a.hid = ws.hbuf;  // the last layer's activations stay readable (tt_stage_offsets)
+    }
+    rc = launch_rowchain(a, D, true, stream);
+  }
+  return rc;
+}
+
 // The forward on a workspace the caller provides (tt_transformer_fwd) or on the library's own
 // scratch array (tt_transformer_fwd_noalloc, which clears the megakernel's counters first).
 int transformer_fwd(const void* weights, const void* x, const uint8_t* mask, void* y,
@@ -437,6 +508,9 @@ int transformer_fwd(const void* weights, const void* x, const uint8_t* mask, voi
     if ((rc = launch_mask_info(mask, ws.info, B, S, stream)) != TT_OK) return rc;
     info = ws.info;
   }
+  if (chains_rows(mask != nullptr, B, S, D, H, F))
+    return forward_chained(wts, lay, (const half*)x, mask, (half*)y, ws, info, B, S, D, H, F, L, causal,
+                           stream);
   // Layer-wise plan: LN2 of every layer and LN1 of layers >= 1 are folded into the projection
   // that follows them (lnfold.hip): the producer of the residual stream (out_proj, ffn_out)
   // writes partial row statistics in its epilogue, and the QKV / ffn_in GEMMs multiply the raw

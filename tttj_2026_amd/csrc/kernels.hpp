@@ -131,6 +131,29 @@ int megakernel_attach_status(void* workspace, int64_t workspace_bytes, int B, in
 // Polls per dependency wait before it gives up, for later launches (< 0: the default).
 void megakernel_set_spin_limit(int64_t limit);
 
+// Row chain of narrow models (rowchain.hip): with `mid`, out_proj ... ffn_out of the layer at w on (x, ctx),
+// then (y == nullptr) LN1 and QKV of the layer at wn, the residual stream stored to xa, or (y) the final
+// norm into y; without it only LN1 and QKV of wn on x.  hid, if given, receives the GELU activations.
+struct ChainArgs {
+  const half *w, *wn;                      // layer bases in the packed weights
+  const half *fw, *fwn;                    // their fragment-order copies (launch_pack_fragments)
+  int64_t off[TT_LAYER_SEGMENTS];
+  const half *fin_g, *fin_b;
+  const half *x, *ctx;
+  half *xa, *q, *hid, *y;                  // q: the TT_EPI_QKV planes
+  const uint8_t* valid;                    // [T] or nullptr
+  int T, S, H, hd, hd_log2, F, ldv;
+  float q_scale;
+};
+// Fragment-order copies of a layer's Wqkv, Wo, W1 and W2 for the row chain, in this order: 1 KiB tiles of
+// 16 rows x 32 columns, lane l's 16 bytes being row l % 16, columns 8 (l / 16) + 0..7.  0 for widths the
+// row chain does not take.
+constexpr int kChainMaxD = 192, kChainMaxF = 1024;
+int64_t chain_fragment_halfs(int64_t D, int64_t F);
+int launch_pack_fragments(const half* w, int64_t stride, const int64_t* off, half* frag, int D, int F, int L,
+                          hipStream_t stream);
+int launch_rowchain(const ChainArgs& a, int d_model, bool mid, hipStream_t stream);
+
 // The whole forward (tt_transformer_fwd's body, forward.hip) on the given workspace; with
 // reset_counters the megakernel plan first clears its dependency counters (a workspace shared
 // with calls of other shapes).
