@@ -1,9 +1,10 @@
 // Row LayerNorm for the pre-LN block stack (norm1 / norm2 / final_norm) on gfx950.
 //
-// One 64-lane wave owns one row of D fp16 values (D <= 8192): every lane loads its 16-byte chunks
-// once into registers, the wave reduces the mean, then the centred second moment (two-pass, fp32),
-// and writes (x - mean) * rsqrt(var + eps) * gamma + beta as fp16.  Rows whose mask byte is zero
-// are written as +0.0 (the final_norm + masked_fill of torch_transformer_benchmark.py:169-171).
+// G lanes own one row of D fp16 values (D <= 8192): a whole wave for D > 256, 32, 16 or 8 lanes for narrower
+// rows, so that no lane is without a 16-byte chunk (one row per wave left 48 of 64 lanes idle at D = 128:
+// 65536 x 128 14.0 -> 6.0 us on MI355X, 30000 x 256 8.0 -> 5.6).  Every lane loads its chunks once into
+// registers, the lanes reduce the mean, then the centred second moment (two-pass, fp32), and write
+// (x - mean) * rsqrt(var + eps) * gamma + beta as fp16.  Rows whose mask byte is zero are written as +0.0 (the final_norm + masked_fill of torch_transformer_benchmark.py:169-171).
 // HBM-bound: 4*D bytes per row (+4*D for gamma/beta, cached).
 #include "common.hpp"
 #include "kernels.hpp"
@@ -19,22 +20,22 @@ struct LnRows {
   half* copy_out;
 };
 
-template <int NV>
+template <int NV, int G = 64>
 __global__ __launch_bounds__(256) void layernorm_kernel(const half* __restrict__ x,
                                                         const half* __restrict__ gamma,
                                                         const half* __restrict__ beta,
                                                         const uint8_t* __restrict__ valid,
                                                         half* __restrict__ y, int rows, int d,
                                                         float eps, LnRows pk) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * (256 / G) + threadIdx.x / G;
+  const int lane = threadIdx.x & (G - 1);
   if (pk.n_dev != nullptr) rows = min(rows, *pk.n_dev);
   if (row >= rows) return;
   const int nch = d >> 3;
   const size_t base = (size_t)row * d;
   const int src = pk.in_row != nullptr ? pk.in_row[row] : row;
   if ((valid != nullptr && valid[row] == 0) || src < 0) {
-    for (int c = lane; c < nch; c += 64) {
+    for (int c = lane; c < nch; c += G) {
       *(uint4*)(y + base + 8 * c) = make_uint4(0, 0, 0, 0);
       if (pk.copy_out != nullptr) *(uint4*)(pk.copy_out + base + 8 * c) = make_uint4(0, 0, 0, 0);
     }
@@ -46,7 +47,7 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const half* __restrict__
   half8 v[NV], g[NV], bt[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int c = lane + 64 * i;
+    const int c = lane + G * i;
     if (c < nch) {
       v[i] = *(const half8*)(x + sbase + 8 * c);
       if (pk.copy_out != nullptr) *(half8*)(pk.copy_out + base + 8 * c) = v[i];
@@ -57,17 +58,17 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const half* __restrict__
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int c = lane + 64 * i;
+    const int c = lane + G * i;
     if (c < nch) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) s += (float)v[i][e];
     }
   }
-  const float mean = wave_sum(s) / (float)d;
+  const float mean = seg_sum<G>(s) / (float)d;
   float q = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int c = lane + 64 * i;
+    const int c = lane + G * i;
     if (c < nch) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
@@ -76,10 +77,10 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const half* __restrict__
       }
     }
   }
-  const float rstd = rsqrtf(wave_sum(q) / (float)d + eps);
+  const float rstd = rsqrtf(seg_sum<G>(q) / (float)d + eps);
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int c = lane + 64 * i;
+    const int c = lane + G * i;
     if (c < nch) {
       half8 o;
 #pragma unroll
@@ -96,19 +97,22 @@ int launch_layernorm_rows(const half* x, const half* gamma, const half* beta, co
   TT_REQUIRE(rows >= 0 && d > 0 && d % 8 == 0 && d <= 8192,
              "layernorm: need d %% 8 == 0 and 0 < d <= 8192 (got d=%d)", d);
   if (rows == 0) return TT_OK;
-  const dim3 grid((rows + 3) / 4), block(256);
-  const int nv = (d / 8 + 63) / 64;
+  const dim3 block(256);
   const LnRows pk{in_row, n_dev, copy_out};
-  if (nv <= 1)
-    hipLaunchKernelGGL(layernorm_kernel<1>, grid, block, 0, stream, x, gamma, beta, valid, y, rows, d, eps, pk);
-  else if (nv <= 2)
-    hipLaunchKernelGGL(layernorm_kernel<2>, grid, block, 0, stream, x, gamma, beta, valid, y, rows, d, eps, pk);
-  else if (nv <= 4)
-    hipLaunchKernelGGL(layernorm_kernel<4>, grid, block, 0, stream, x, gamma, beta, valid, y, rows, d, eps, pk);
-  else if (nv <= 8)
-    hipLaunchKernelGGL(layernorm_kernel<8>, grid, block, 0, stream, x, gamma, beta, valid, y, rows, d, eps, pk);
-  else
-    hipLaunchKernelGGL(layernorm_kernel<16>, grid, block, 0, stream, x, gamma, beta, valid, y, rows, d, eps, pk);
+  auto run = [&](auto kernel, int lanes) {
+    const int per = 256 / lanes;
+    hipLaunchKernelGGL(kernel, dim3((rows + per - 1) / per), block, 0, stream, x, gamma, beta, valid, y, rows, d,
+                       eps, pk);
+  };
+  const int nch = d / 8, nv = (nch + 63) / 64;
+  if (nch <= 8) run(layernorm_kernel<1, 8>, 8);
+  else if (nch <= 16) run(layernorm_kernel<1, 16>, 16);
+  else if (nch <= 32) run(layernorm_kernel<1, 32>, 32);
+  else if (nv <= 1) run(layernorm_kernel<1>, 64);
+  else if (nv <= 2) run(layernorm_kernel<2>, 64);
+  else if (nv <= 4) run(layernorm_kernel<4>, 64);
+  else if (nv <= 8) run(layernorm_kernel<8>, 64);
+  else run(layernorm_kernel<16>, 64);
   return launch_status("layernorm_kernel");
 }
 
