@@ -410,10 +410,11 @@ static int forward_packed(const half* wts, const Layout& lay, const half* x, con
 }
 
 // Layer-wise forward of a narrow model: LN1 + QKV of layer 0, then per layer the attention and the row
-// chain up to the next layer's QKV projection or the final norm (2 L + 1 launches, one more with a mask).
+// chain up to the next layer's QKV projection or the final norm (2 L + 1 launches; the first one also makes
+// the mask summary).
 static int forward_chained(const half* wts, const Layout& lay, const half* x, const uint8_t* mask, half* y,
-                           const Workspace& ws, const int32_t* info, int B, int S, int D, int H, int F,
-                           int L, int causal, hipStream_t stream) {
+                           const Workspace& ws, int B, int S, int D, int H, int F, int L, int causal,
+                           hipStream_t stream) {
   const int hd = D / H;
   const size_t plane = (size_t)B * S * D;
   ChainArgs a{};
@@ -424,6 +425,9 @@ static int forward_chained(const half* wts, const Layout& lay, const half* x, co
   a.xa = ws.xa;
   a.q = ws.qkv;
   a.valid = mask;
+  a.info = ws.info;
+  a.info_blocks = mask != nullptr ? B : 0;
+  const int32_t* info = mask != nullptr ? ws.info : nullptr;
   a.T = B * S;
   a.S = S;
   a.H = H;
@@ -504,13 +508,12 @@ int transformer_fwd(const void* weights, const void* x, const uint8_t* mask, voi
     return forward_packed(wts, lay, (const half*)x, mask, (half*)y, ws, ws.info, B, S, D, H, F, L,
                           causal, stream);
   }
+  if (chains_rows(mask != nullptr, B, S, D, H, F))
+    return forward_chained(wts, lay, (const half*)x, mask, (half*)y, ws, B, S, D, H, F, L, causal, stream);
   if (mask != nullptr) {
     if ((rc = launch_mask_info(mask, ws.info, B, S, stream)) != TT_OK) return rc;
     info = ws.info;
   }
-  if (chains_rows(mask != nullptr, B, S, D, H, F))
-    return forward_chained(wts, lay, (const half*)x, mask, (half*)y, ws, info, B, S, D, H, F, L, causal,
-                           stream);
   // Layer-wise plan: LN2 of every layer and LN1 of layers >= 1 are folded into the projection
   // that follows them (lnfold.hip): the producer of the residual stream (out_proj, ffn_out)
   // writes partial row statistics in its epilogue, and the QKV / ffn_in GEMMs multiply the raw

@@ -142,6 +142,8 @@ struct ChainArgs {
   const half *x, *ctx;
   half *xa, *q, *hid, *y;                  // q: the TT_EPI_QKV planes
   const uint8_t* valid;                    // [T] or nullptr
+  int32_t* info;                           // launch_mask_info's output, written by the first launch for
+  int info_blocks;                         //   this many sequences (0: no mask)
   int T, S, H, hd, hd_log2, F, ldv;
   float q_scale;
 };

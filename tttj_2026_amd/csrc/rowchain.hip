@@ -78,6 +78,37 @@ __global__ __launch_bounds__(kChainThreads, 2) void rowchain_kernel(ChainArgs a)
   const int col = lane & 15, g4 = lane >> 4;
   const int T = a.T, S = a.S;
   const bool last = MID && a.y != nullptr;
+  const int nblocks = (int)gridDim.x - (MID ? 0 : a.info_blocks);  // blocks with row tiles
+  if (!MID && (int)blockIdx.x >= nblocks) {
+    // One block per sequence behind them: the mask summary the attention launches read (as
+    // mask_info_kernel), beside the row tiles instead of in a launch of its own.
+    const int b = blockIdx.x - nblocks;
+    int end = 0, count = 0;
+    for (int s = tid; s < S; s += NT)
+      if (a.valid[(size_t)b * S + s] != 0) {
+        end = s + 1;
+        ++count;
+      }
+    __shared__ int s_end[8], s_count[8];
+    for (int off = 32; off > 0; off >>= 1) {
+      end = max(end, __shfl_xor(end, off));
+      count += __shfl_xor(count, off);
+    }
+    if (lane == 0) {
+      s_end[wave] = end;
+      s_count[wave] = count;
+    }
+    __syncthreads();
+    if (tid == 0) {
+      for (int w = 1; w < 8; ++w) {
+        end = max(end, s_end[w]);
+        count += s_count[w];
+      }
+      a.info[b] = end;
+      a.info[a.info_blocks + b] = count == end;
+    }
+    return;
+  }
 
   // Loads the first GEMM waits for come first: the rows, then its weights, then the rest.
   constexpr int XL = (R * CH + NT - 1) / NT;
@@ -97,7 +128,7 @@ __global__ __launch_bounds__(kChainThreads, 2) void rowchain_kernel(ChainArgs a)
   // Past the last tile: INT_MAX (later rounds lie past it too).
   auto tile_of = [&](int round) {
     if (!KEEP) return INT_MAX;
-    const int g = gridDim.x, t = round * g + (int)((blockIdx.x + 5u * round) % (unsigned)g);
+    const int g = nblocks, t = round * g + (int)((blockIdx.x + 5u * round) % (unsigned)g);
     return t < ntiles ? t : INT_MAX;
   };
   load_rows(blockIdx.x);
@@ -487,6 +518,7 @@ static int run_chain(const ChainArgs& a, hipStream_t stream) {
     return fail(TT_ERR_HIP, "hipFuncSetAttribute(rowchain): %s", hipGetErrorString(attr));
   int blocks = (a.T + 16 * RT - 1) / (16 * RT);
   if (KEEP) blocks = std::min(blocks, kChainBlocks);
+  if (!MID) blocks += a.info_blocks;
   hipLaunchKernelGGL((rowchain_kernel<D, RT, MID, KEEP>), dim3(blocks), dim3(kChainThreads),
                      chain_lds_bytes(D, RT, MID ? a.F : 0), stream, a);
   return launch_status("rowchain_kernel");
