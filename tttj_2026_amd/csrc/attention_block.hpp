@@ -28,6 +28,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "kernels.hpp"
 
 #include <mutex>
 
@@ -69,6 +70,12 @@ __device__ __forceinline__ float xhalf_sum(float v) {  // sum over lanes l and l
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// v if bit `bit` of `allowed` is set, else -inf: a sign-extended bit and one bitwise select (two
+// instructions; compare and conditional move take three).
+__device__ __forceinline__ float keep_or_ninf(float v, uint32_t allowed, int bit) {
+  const uint32_t t = (uint32_t)((int32_t)(allowed << (31 - bit)) >> 31);
+  return __uint_as_float((t & __float_as_uint(v)) | (~t & 0xff800000u));
+}
 
 // Arguments shared by every attention block of one launch (see attention_block).
 struct AttnArgs {
@@ -96,7 +103,9 @@ struct AttnArgs {
 // in-flight copies from the tile being read and waits for all of them before its first MFMA).
 // POLICY is the cache policy of the Q, K and V^T loads (kLoadDevice when other workgroups of the
 // same launch wrote them).
-template <int HD, bool CAUSAL, int POLICY = kLoadDefault, bool RING3 = false>
+// NSPLIT > 1: the block has NSPLIT groups of four waves; group g takes key tiles g, g + NSPLIT, ... with its
+// own ring of two, and at the end group 0 merges the groups' (O, max, sum) through LDS, in group order.
+template <int HD, bool CAUSAL, int POLICY = kLoadDefault, bool RING3 = false, int NSPLIT = 1>
 __device__ __forceinline__ void attention_block(const AttnArgs& a, int bh, int qt, int kv_end,
                                                 bool prefix, half* sk_base, half* sv_base) {
   static_assert(HD == 32 || HD == 64 || HD == 128 || HD == 256, "MFMA attention head_dim");
@@ -108,8 +117,10 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, int bh, int q
   constexpr int VCOPIES = HD * kBKV * 2 / 1024 / 4;  // V^T copies per wave per tile
   constexpr float kLazy = 8.0f;    // log2 growth of the row max that forces a rescale
 
-  half (*sk)[kBKV * HD] = reinterpret_cast<half (*)[kBKV * HD]>(sk_base);
-  half (*sv)[HD * kBKV] = reinterpret_cast<half (*)[HD * kBKV]>(sv_base);
+  static_assert(NSPLIT == 1 || !RING3, "split groups use the ring of two");
+  const int grp = NSPLIT == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  half (*sk)[kBKV * HD] = reinterpret_cast<half (*)[kBKV * HD]>(sk_base + grp * (2 * kBKV * HD));
+  half (*sv)[HD * kBKV] = reinterpret_cast<half (*)[HD * kBKV]>(sv_base + grp * (2 * kBKV * HD));
   const half* __restrict__ Q = a.Q;
   const half* __restrict__ K = a.K;
   const half* __restrict__ Vt = a.Vt;
@@ -118,7 +129,7 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, int bh, int q
   const int S = a.S, H = a.H;
   const float scale_log2 = a.scale_log2;
   const int b = bh / H, h = bh - b * H;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = NSPLIT == 1 ? threadIdx.x : threadIdx.x & 255, lane = tid & 63;  // within the group
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hf = lane >> 5, col = lane & 31;
   const int ldv = round_up(S, kBKV);
@@ -225,31 +236,34 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, int bh, int q
   };
   int mcur = 0, mnext = 0;
   if (ntiles > 0) {
-    issue_tile(0, 0);
-    if (!r3 && keymask) mcur = mask_byte(0);
+    if (NSPLIT == 1 || grp < ntiles) issue_tile(grp * kBKV, 0);
+    if (!r3 && keymask) mcur = mask_byte(grp * kBKV);
     // Both first tiles land before the loop: with copies still in flight on entry, the compiler
     // adds a wait for the next tile's copies before every tile's first MFMA.
     if (r3 && ntiles > 1) issue_tile(kBKV, 1);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (kBKV > S) {
-      clear_vt_tail(0, 0);
+    if (NSPLIT * kBKV > S) {  // a group's first tile is the partial last one (t0 + 64 > S > t0)
+      if (NSPLIT == 1 || (grp < ntiles && (grp + 1) * kBKV > S)) clear_vt_tail(grp * kBKV, 0);
       __syncthreads();
     }
   }
-  for (int t = 0; t < ntiles; ++t) {
-    const int st = r3 ? t % 3 : (t & 1);
+  // Rounds of one tile per group (barriers are the block's, so every group runs every round).
+  const int rounds = (ntiles + NSPLIT - 1) / NSPLIT;
+  for (int round = 0; round < rounds; ++round) {
+    const int t = NSPLIT * round + grp;
+    const int st = r3 ? t % 3 : (round & 1);
     const int t0 = t * kBKV;
-    if (!r3 && t + 1 < ntiles) {
-      issue_tile(t0 + kBKV, st ^ 1);
-      if (keymask) mnext = mask_byte(t0 + kBKV);
+    if (!r3 && t + NSPLIT < ntiles) {
+      issue_tile(t0 + NSPLIT * kBKV, st ^ 1);
+      if (keymask) mnext = mask_byte(t0 + NSPLIT * kBKV);
     }
     // Ring of three: the copies of tile t + 2 go to the buffer tile t - 1 used.
     if (r3) {
       if (keymask) mcur = mask_byte(t0);
       if (t + 2 < ntiles) issue_tile(t0 + 2 * kBKV, st == 0 ? 2 : st - 1);
     }
-    if (wave_active && t0 < wave_end) {
+    if (wave_active && t0 < wave_end) {  // (t0 < wave_end implies t < ntiles)
       floatx16 s[2];
       // The S^T MFMAs issue at raised wave priority: the SIMD's other waves are mostly in their
       // softmax (vector ALU), so a wave that reaches its MFMAs gets the matrix unit first
@@ -287,7 +301,7 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, int bh, int q
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
           for (int j = 0; j < 16; ++j)
-            if (!((allowed >> (16 * kb + j)) & 1u)) s[kb][j] = -INFINITY;
+            s[kb][j] = keep_or_ninf(s[kb][j], allowed, 16 * kb + j);
       }
       float mx = s[0][0];
 #pragma unroll
@@ -343,7 +357,7 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, int bh, int q
       }
     }
     if (!r3) mcur = mnext;
-    if (t + 1 < ntiles) {
+    if (round + 1 < rounds) {
       const int sn = r3 ? (st == 2 ? 0 : st + 1) : (st ^ 1);
       if (r3 && t + 2 < ntiles) {
         // The next tile's copies have landed (those of tile t + 2, issued after them, may stay
@@ -355,10 +369,44 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, int bh, int q
         __builtin_amdgcn_s_waitcnt(0);  // the next tile's copies have landed ...
         __syncthreads();                // ... and every wave is done with this one
       }
-      if (t0 + 2 * kBKV > S) {        // next tile is the partial last one
-        clear_vt_tail(t0 + kBKV, sn);
+      if (NSPLIT * (round + 2) * kBKV > S) {  // a next tile is the partial last one
+        const int tn = t0 + NSPLIT * kBKV;
+        if (NSPLIT == 1 || (tn < ntiles * kBKV && tn + kBKV > S)) clear_vt_tail(tn, sn);
         __syncthreads();
       }
+    }
+  }
+
+  if constexpr (NSPLIT > 1) {
+    // [group - 1][wave][value][lane]: the O values, the reference max and this lane's half of the sum
+    constexpr int NV = DB * 16 + 2;
+    float* const mrg = reinterpret_cast<float*>(sk_base);
+    __syncthreads();  // every group is done with its tiles
+    if (grp > 0) {
+      float* p = mrg + (size_t)((grp - 1) * 4 + wave) * NV * 64 + lane;
+#pragma unroll
+      for (int i = 0; i < DB; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) p[(i * 16 + e) * 64] = o[i][e];
+      p[(NV - 2) * 64] = m_ref;
+      p[(NV - 1) * 64] = l_run;
+    }
+    __syncthreads();
+    if (grp > 0) return;
+#pragma unroll 1
+    for (int gi = 0; gi < NSPLIT - 1; ++gi) {
+      const float* p = mrg + (size_t)(gi * 4 + wave) * NV * 64 + lane;
+      const float m_g = p[(NV - 2) * 64], l_g = p[(NV - 1) * 64];
+      const float m_new = fmaxf(m_ref, m_g);
+      // a part without a valid key (max -inf) holds zeros and weighs 0
+      const float c0 = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_ref - m_new);
+      const float c1 = m_g == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_g - m_new);
+      m_ref = m_new;
+      l_run = l_run * c0 + l_g * c1;
+#pragma unroll
+      for (int i = 0; i < DB; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[i][e] = o[i][e] * c0 + p[(i * 16 + e) * 64] * c1;
     }
   }
 
@@ -394,14 +442,14 @@ inline bool attention_ring3(int hd, int seq) { return attention_ring3_hd(hd) && 
 
 // Standalone launch: one block per (b, h, 128-query tile).  `info` (or nullptr without a mask)
 // holds kv_end per sequence and whether its valid keys form a prefix (mask_info_kernel).
-template <int HD, bool CAUSAL, bool RING3>
-__global__ __launch_bounds__(256) void attention_kernel(AttnArgs a, const int32_t* __restrict__ info) {
+template <int HD, bool CAUSAL, bool RING3, int NSPLIT = 1>
+__global__ __launch_bounds__(256 * NSPLIT) void attention_kernel(AttnArgs a, const int32_t* __restrict__ info) {
   // Dynamic LDS: with statically declared tiles the compiler makes the first K-fragment read of
   // every tile wait (vmcnt(0)) for the next tile's in-flight global -> LDS copies, serialising
   // the prefetch; from the dynamic area it relies on the explicit waits, as intended.
   extern __shared__ __align__(16) half att_lds[];
   half* sk = att_lds;
-  half* sv = att_lds + (RING3 ? 3 : 2) * kBKV * HD;
+  half* sv = att_lds + (RING3 ? 3 : 2 * NSPLIT) * kBKV * HD;
   const int BH = a.B * a.H;
   const int nqt = (a.S + kBQ - 1) / kBQ;
   const int bh = blockIdx.x % BH;
@@ -424,7 +472,7 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgs a, const int32_
     constexpr int CPR = HD / 8;  // 16-byte chunks per context row
     const size_t D = (size_t)a.H * HD;
     const int h = bh - b * a.H;
-    for (int e = threadIdx.x; e < kBQ * CPR; e += 256) {
+    for (int e = threadIdx.x; e < kBQ * CPR; e += 256 * NSPLIT) {
       const int q = q0 + e / CPR;
       if (q < a.S)
         *(u32x4*)(a.ctx + ((size_t)b * a.S + q) * D + (size_t)h * HD + 8 * (e % CPR)) =
@@ -432,36 +480,57 @@ __global__ __launch_bounds__(256) void attention_kernel(AttnArgs a, const int32_
     }
     return;
   }
-  attention_block<HD, CAUSAL, kLoadDefault, RING3>(a, bh, qt, kv_end, prefix, sk, sv);
+  attention_block<HD, CAUSAL, kLoadDefault, RING3, NSPLIT>(a, bh, qt, kv_end, prefix, sk, sv);
 }
 
-constexpr size_t attention_lds_bytes(int hd, bool ring3 = false) {
-  return 2 * (size_t)(ring3 ? 3 : 2) * kBKV * hd * sizeof(half);
+constexpr size_t attention_lds_bytes(int hd, bool ring3 = false, int nsplit = 1) {
+  const size_t tiles = 2 * (size_t)(ring3 ? 3 : 2 * nsplit) * kBKV * hd * sizeof(half);
+  const size_t merge = (size_t)(nsplit - 1) * 256 * (hd / 2 + 2) * sizeof(float);
+  return tiles > merge ? tiles : merge;
 }
 
-// Host side: one launch of attention_kernel<HD, CAUSAL, RING3> over every (b, h, query tile);
+// Whether two groups of waves share a block's key tiles (NSPLIT 2).  A small grid's time is the chain of key tiles
+// of its longest blocks, each tile the latency of one wave per SIMD: with fewer blocks than fill the chip's
+// resident slots and at least 16 tiles, two waves per SIMD on alternate tiles shorten it, in spite of the merge at
+// the end.  A causal grid is still bound by its longest blocks at two blocks per CU, if they have 24 tiles and
+// more; at head_dim 32 the split pays up to there either way.  Measured on MI355X, one group -> two: head_dim
+// 128, 32 blocks of 16 tiles 25.0 -> 21.3 us, 256 of 32 (causal) 44.8 -> 36.1, 384 of 24 (causal) 40.6 -> 34.6,
+// but 53.9 -> 61.5 non-causal and 512 of 16 (causal) 32.0 -> 35.1; head_dim 64, 128 of 64 53 -> 39, 256 of 32
+// 29.3 -> 23.4; head_dim 32, 512 of 64 46 -> 37 (causal) and 62 -> 54.  Four groups were no better (head_dim 64
+// spills; head_dim 32 within 10% either way).
+inline bool attention_split(int hd, bool causal, long blocks, int tiles, int cus) {
+  if (hd > 128 || tiles < 16 || blocks > 2L * cus) return false;
+  return blocks <= cus || hd == 32 || (causal && tiles >= 24);
+}
+
+// Host side: one launch of attention_kernel<HD, CAUSAL, RING3, NSPLIT> over every (b, h, query tile);
 // the dynamic LDS limit is raised once per instantiation (above 64 KiB for HD 256).
-template <int HD, bool CAUSAL, bool RING3>
+template <int HD, bool CAUSAL, bool RING3, int NSPLIT = 1>
 int launch_attention_ring(const AttnArgs& args, const int32_t* info, hipStream_t stream) {
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
   std::call_once(once, [] {
-    attr = hipFuncSetAttribute((const void*)attention_kernel<HD, CAUSAL, RING3>,
+    attr = hipFuncSetAttribute((const void*)attention_kernel<HD, CAUSAL, RING3, NSPLIT>,
                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)attention_lds_bytes(HD, RING3));
+                               (int)attention_lds_bytes(HD, RING3, NSPLIT));
   });
   if (attr != hipSuccess)
     return fail(TT_ERR_HIP, "hipFuncSetAttribute(attention hd %d): %s", HD, hipGetErrorString(attr));
   const long blocks = (long)args.B * args.H * ((args.S + kBQ - 1) / kBQ);
   TT_REQUIRE(blocks < (1L << 31), "attention: grid too large");
-  hipLaunchKernelGGL((attention_kernel<HD, CAUSAL, RING3>), dim3((unsigned)blocks), dim3(256),
-                     attention_lds_bytes(HD, RING3), stream, args, info);
+  hipLaunchKernelGGL((attention_kernel<HD, CAUSAL, RING3, NSPLIT>), dim3((unsigned)blocks),
+                     dim3(256 * NSPLIT), attention_lds_bytes(HD, RING3, NSPLIT), stream, args, info);
   return launch_status("attention_kernel");
 }
 
-// The key-tile ring chosen for the sequence length.
+// The key-tile ring and split chosen for the shape.
 template <int HD, bool CAUSAL>
 int launch_attention_hd(const AttnArgs& args, const int32_t* info, hipStream_t stream) {
+  if constexpr (HD <= 128) {
+    const long blocks = (long)args.B * args.H * ((args.S + kBQ - 1) / kBQ);
+    if (attention_split(HD, CAUSAL, blocks, (args.S + kBKV - 1) / kBKV, device_cus()))
+      return launch_attention_ring<HD, CAUSAL, false, 2>(args, info, stream);
+  }
   if constexpr (attention_ring3_hd(HD)) {
     if (attention_ring3(HD, args.S)) return launch_attention_ring<HD, CAUSAL, true>(args, info, stream);
   }

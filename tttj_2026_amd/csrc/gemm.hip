@@ -83,7 +83,7 @@ static int pick_tile(int m, int n, int k, int mode, int cus, bool packed = false
   return 4;  // 64x64: every N that is a multiple of 64
 }
 
-static int device_cus() {
+int device_cus() {
   static int cus = 0;
   if (cus == 0) {
     int dev = 0;

@@ -36,6 +36,8 @@ struct EpiArgs {
   const int2* rowmap;
 };
 
+int device_cus();  // compute units of the current device
+
 int launch_layernorm(const half* x, const half* gamma, const half* beta, const uint8_t* valid,
                      half* y, int rows, int d, float eps, hipStream_t stream);
 // LayerNorm over packed variable-length rows: output row r reads input row in_row[r] (r itself
