@@ -88,23 +88,31 @@ __device__ __forceinline__ void epilogue4(const EpiArgs& ep, int m, int n, const
     *(half4*)dst = hv;
   }
 }
+
 // Narrow-tile GEMM for grids that would leave most CUs idle (few tokens): 32 x 32 output tiles, so
 // four times as many blocks as 64 x 64 tiles pull operands (each CU's streaming rate is set by the
-// bytes it keeps in flight), with the K range split over the block's NW waves.  Each wave loads
-// its W and X fragments straight into registers (lane l: row l % 32, 8 K values at 8 (l / 32)),
-// NPF K steps ahead, and accumulates one 32 x 32 MFMA tile; the NW partial tiles are summed in
-// LDS in wave order (deterministic) and the epilogue runs 4 outputs per thread on the first 256
-// threads.  Long K (few blocks, each streaming many bytes) uses 8 waves with 8 steps per buffer,
-// so a block keeps 128 KiB of operands in flight.
-constexpr int kNarrow = 32;
+// bytes it keeps in flight), with the K range dealt to the block's NW waves in 64-wide slices.  Each wave copies
+// its slices (32 X rows and 32 W rows of 128 bytes) from global memory straight into its own part of LDS, two
+// slices in flight, and accumulates one 32 x 32 MFMA tile from it; no wave reads another's copies, so there is no
+// barrier before the NW partial tiles are summed in wave order (deterministic).  The epilogue runs 4 outputs per
+// thread on the first 256 threads.  Copies read 8 rows x 128 bytes an instruction (18 cycles of the CU's address
+// unit); fragments loaded straight into registers, 32 rows x 16 bytes twice, took 64, the bound of this kernel at
+// long K.  Measured on MI355X, registers -> LDS: 512 x 768 x 256 4.7 -> 4.1 us, 512 x 256 x 1024 6.2 -> 4.6,
+// 21 x 320 x 1280 8.9 -> 4.7, 128 x 1024 x 4096 17.0 -> 7.6, 396 x 768 x 3072 25.3 -> 12.2 (a launch by itself ~3.5).
+// Long K uses 8 waves, so that a block keeps 128 KiB of operands in flight.
 //
 // RAG: N (for the QKV projection each of its three parts) and K are multiples of 8 only.  A part's last
 // column tile is then partial: W rows past the part are clamped to its last one and their outputs not
-// stored.  K is dealt to the waves in whole 16-wide steps; 8-value chunks at or past K read as zero.
-template <int MODE, int NW, int NPF, bool RAG>
+// stored.  8-value chunks at or past K are replaced by zeros when they are read from LDS.
+constexpr int kNarrow = 32;
+constexpr int kNarrowSlice = 2 * kNarrow * kBK;  // halfs: X rows 0 .. 31, W rows 32 .. 63
+constexpr size_t narrow_lds_bytes(int nw) { return (size_t)nw * 2 * kNarrowSlice * sizeof(half); }
+
+template <int MODE, int NW, bool RAG>
 __global__ __launch_bounds__(64 * NW) void gemm_narrow_kernel(const half* __restrict__ X,
                                                               const half* __restrict__ W, int M,
                                                               int N, int K, EpiArgs ep) {
+  extern __shared__ __align__(16) half lds[];
   const int tiles_n = column_tiles<kNarrow, MODE, RAG>(N);
   const int tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
   const int m0 = tm * kNarrow;
@@ -115,21 +123,33 @@ __global__ __launch_bounds__(64 * NW) void gemm_narrow_kernel(const half* __rest
     n0 = part * width + (tn - part * per) * kNarrow;
     n_end = (part + 1) * width;
   }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int r = lane & 31, kh = 8 * (lane >> 5);
-  const half* xr = X + (size_t)min(m0 + r, M - 1) * K + kh;
-  const half* wr = W + (size_t)(RAG ? min(n0 + r, n_end - 1) : n0 + r) * K + kh;
-  // K steps of this wave (K % (16 NW) == 0 unless RAG, whose last waves may have fewer or none)
-  int steps = K / 16 / NW;
-  int kbeg = wave * steps * 16;
-  if constexpr (RAG) {
-    // The step count differs between waves, and MFMAs ignore the lane mask: it is made provably
-    // uniform so that a wave with fewer steps branches over them.
-    const int all = (K + 15) / 16, per = (all + NW - 1) / NW;
-    const int first = __builtin_amdgcn_readfirstlane(wave) * per;
-    kbeg = first * 16;
-    steps = max(0, min(per, all - first));
+  // wave index provably uniform: MFMAs ignore the lane mask, so a wave with fewer slices must branch
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 31, hi = lane >> 5;
+  half* const ring = lds + wave * (2 * kNarrowSlice);
+  // Copy c fills rows 8 c .. 8 c + 7 of the slice: lane l row 8 c + l / 8, physical chunk l % 8, which holds
+  // logical chunk (l % 8) ^ bits 1-3 of the row (the layout of gemm_kernel's direct copies).
+  const int lrow = lane >> 3;
+  const half* src[8];
+  int col[2];  // the lane's first column in a slice, for even and odd copies
+#pragma unroll
+  for (int c = 0; c < 2; ++c) col[c] = 8 * ((lane & 7) ^ ((c << 2) | (lrow >> 1)));
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    const int row = 8 * (c & 3) + lrow;
+    src[c] = c < 4 ? X + (size_t)min(m0 + row, M - 1) * K
+                   : W + (size_t)(RAG ? min(n0 + row, n_end - 1) : n0 + row) * K;
   }
+  auto copy = [&](int s, int slot) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const int k = s * kBK + col[c & 1];
+      lds_copy16(src[c] + (RAG && k >= K ? 0 : k), ring + slot * kNarrowSlice + c * 512);
+    }
+  };
+  // slices wave, wave + NW, ...
+  const int all = RAG ? (K + kBK - 1) / kBK : K / kBK;
+  const int mine = (all - wave + NW - 1) / NW;
   // epilogue mapping (below): thread -> row ml, 4 columns nl; 8 aligned threads per row
   const int et = threadIdx.x & 255;
   const int ml = et >> 3, nl = 4 * (et & 7);
@@ -138,75 +158,84 @@ __global__ __launch_bounds__(64 * NW) void gemm_narrow_kernel(const half* __rest
   floatx16 acc;
 #pragma unroll
   for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-  half8 a[2][NPF], b[2][NPF];
-  auto load = [&](int buf, int s0) {
+  if (mine > 0) copy(wave, 0);
+  if (mine > 1) copy(wave + NW, 1);
+  for (int j = 0; j < mine; ++j) {
+    const int s = wave + NW * j;
+    if (j + 1 < mine) wait_vmcnt<8>();  // this slice's copies have landed (the next one's 8 may not have)
+    else wait_vmcnt<0>();
+    asm volatile("" ::: "memory");
+    const half* st = ring + (j & 1) * kNarrowSlice;
+    half8 a[4], b[4];
 #pragma unroll
-    for (int j = 0; j < NPF; ++j) {
-      const int k = kbeg + 16 * min(s0 + j, steps - 1);  // past the end: reload the last step
+    for (int kk = 0; kk < 4; ++kk) {
+      const int pc = ((2 * kk + hi) ^ ((r >> 1) & 7)) * 8;
+      b[kk] = *(const half8*)(st + r * kBK + pc);
+      a[kk] = *(const half8*)(st + (kNarrow + r) * kBK + pc);
       if constexpr (RAG) {
-        const bool in = k >= 0 && k + kh < K;  // 8 values of one row, all inside K or none
-        const half8 wv = *(const half8*)(in ? wr + k : wr - kh);
-        const half8 xv = *(const half8*)(in ? xr + k : xr - kh);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          a[buf][j][e] = in ? wv[e] : (half)0.f;
-          b[buf][j][e] = in ? xv[e] : (half)0.f;
-        }
-      } else {
-        a[buf][j] = *(const half8*)(wr + k);
-        b[buf][j] = *(const half8*)(xr + k);
+        const bool in = s * kBK + 16 * kk + 8 * hi < K;  // 8 values of one row, all inside K or none
+        const u32x4 wa = __builtin_bit_cast(u32x4, a[kk]), wb = __builtin_bit_cast(u32x4, b[kk]);
+        a[kk] = __builtin_bit_cast(half8, u32x4{in ? wa[0] : 0u, in ? wa[1] : 0u, in ? wa[2] : 0u, in ? wa[3] : 0u});
+        b[kk] = __builtin_bit_cast(half8, u32x4{in ? wb[0] : 0u, in ? wb[1] : 0u, in ? wb[2] : 0u, in ? wb[3] : 0u});
       }
     }
-  };
-  auto mma = [&](int buf, int s0) {
 #pragma unroll
-    for (int j = 0; j < NPF; ++j)
-      if (s0 + j < steps) acc = mfma32x32x16(a[buf][j], b[buf][j], acc);
-  };
-  // Two buffers, alternated by a loop unrolled twice (register arrays need compile-time indices).
-  load(0, 0);
-  for (int s0 = 0; s0 < steps; s0 += 2 * NPF) {
-    if (s0 + NPF < steps) load(1, s0 + NPF);
-    mma(0, s0);
-    if (s0 + NPF >= steps) break;
-    if (s0 + 2 * NPF < steps) load(0, s0 + 2 * NPF);
-    mma(1, s0 + NPF);
+    for (int kk = 0; kk < 4; ++kk) acc = mfma32x32x16(a[kk], b[kk], acc);
+    if (j + 2 < mine) {
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the slice has been read ...
+      asm volatile("" ::: "memory");
+      copy(s + 2 * NW, j & 1);             // ... and its place is free
+    }
   }
   // acc[4g + e] = C[m0 + r][n0 + 8g + 4 (lane / 32) + e]
-  __shared__ __align__(16) float part[NW][kNarrow][kNarrow];
+  // (a wave's partial tile takes the place of its own slices)
+  auto part = [&](int w) { return reinterpret_cast<float*>(lds + w * (2 * kNarrowSlice)); };
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  asm volatile("" ::: "memory");
 #pragma unroll
   for (int g = 0; g < 4; ++g)
-    *(floatx4*)&part[wave][r][8 * g + 4 * (lane >> 5)] =
+    *(floatx4*)(part(wave) + r * kNarrow + 8 * g + 4 * hi) =
         floatx4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
   __syncthreads();
   if (threadIdx.x >= 256 || m0 + ml >= M) return;
   float sum[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    float v = part[0][ml][nl + e];
+    float v = part(0)[ml * kNarrow + nl + e];
 #pragma unroll
-    for (int w = 1; w < NW; ++w) v += part[w][ml][nl + e];
+    for (int w = 1; w < NW; ++w) v += part(w)[ml * kNarrow + nl + e];
     sum[e] = v;
   }
   if (RAG && n0 + nl >= n_end) return;
   epilogue4<MODE, 8>(ep, m0 + ml, n0 + nl, sum, pre);
 }
 
-// Long K: 8 waves (more than two 4-step buffers per wave at 4 waves).
-template <bool RAG>
-static bool narrow_long_k(int k) { return (RAG || k % 128 == 0) && k / 64 > 8; }
+// 8 waves above K = 512 (more than the two slices per wave that 4 waves hold at once).
+static bool narrow_long_k(int k) { return k > 512; }
+
+template <int MODE, int NW, bool RAG>
+static int launch_narrow_waves(const half* x, const half* w, int m, int n, int k, const EpiArgs& ep,
+                               hipStream_t stream) {
+  static std::once_flag once;
+  static hipError_t attr = hipSuccess;
+  std::call_once(once, [] {
+    attr = hipFuncSetAttribute((const void*)gemm_narrow_kernel<MODE, NW, RAG>,
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)narrow_lds_bytes(NW));
+  });
+  if (attr != hipSuccess)
+    return fail(TT_ERR_HIP, "hipFuncSetAttribute(gemm_narrow): %s", hipGetErrorString(attr));
+  const long blocks = (long)((m + kNarrow - 1) / kNarrow) * column_tiles<kNarrow, MODE, RAG>(n);
+  TT_REQUIRE(blocks < (1L << 31), "linear: grid too large");
+  hipLaunchKernelGGL((gemm_narrow_kernel<MODE, NW, RAG>), dim3((unsigned)blocks), dim3(64 * NW),
+                     narrow_lds_bytes(NW), stream, x, w, m, n, k, ep);
+  return launch_status("gemm_narrow_kernel");
+}
 
 template <int MODE, bool RAG>
 static int launch_narrow_mode(const half* x, const half* w, int m, int n, int k, const EpiArgs& ep,
                               hipStream_t stream) {
-  const long blocks = (long)((m + kNarrow - 1) / kNarrow) * column_tiles<kNarrow, MODE, RAG>(n);
-  TT_REQUIRE(blocks < (1L << 31), "linear: grid too large");
-  const dim3 grid((unsigned)blocks);
-  if (narrow_long_k<RAG>(k))
-    hipLaunchKernelGGL((gemm_narrow_kernel<MODE, 8, 8, RAG>), grid, dim3(512), 0, stream, x, w, m, n, k, ep);
-  else
-    hipLaunchKernelGGL((gemm_narrow_kernel<MODE, 4, 4, RAG>), grid, dim3(256), 0, stream, x, w, m, n, k, ep);
-  return launch_status("gemm_narrow_kernel");
+  return narrow_long_k(k) ? launch_narrow_waves<MODE, 8, RAG>(x, w, m, n, k, ep, stream)
+                          : launch_narrow_waves<MODE, 4, RAG>(x, w, m, n, k, ep, stream);
 }
 
 }  // namespace tt
