@@ -34,16 +34,18 @@ static int run_mode(int tile, const half* x, const half* w, int m, int n, int k,
     case 8: return run_tile<128, 64, MODE, 1>(x, w, m, n, k, ep, stream);
     case 9: return run_tile<256, 128, MODE, 1>(x, w, m, n, k, ep, stream);
     case 10: return run_tile<256, 128, MODE, 0, 8>(x, w, m, n, k, ep, stream);
+    case 11: return run_tile<64, 64, MODE, 1>(x, w, m, n, k, ep, stream);
     default: return run_tile<64, 64, MODE, 0>(x, w, m, n, k, ep, stream);
   }
 }
 
 // index 0: 256 x 256 on 8 waves; index 5: 32 x 32 narrow tiles (gemm_narrow_kernel), chosen for
 // grids that leave most CUs idle; indices 6-9: 128 x 256, 128 x 128, 128 x 64, 256 x 128 on the
-// register path; index 10: 256 x 128 on 8 waves with a three-stage ring
+// register path; index 10: 256 x 128 on 8 waves with a three-stage ring; index 11: 64 x 64 on the
+// register path
 static const TileCfg kTiles[] = {{256, 256}, {256, 128}, {128, 128}, {128, 64}, {64, 64},
                                  {32, 32},   {128, 256}, {128, 128}, {128, 64}, {256, 128},
-                                 {256, 128}};
+                                 {256, 128}, {64, 64}};
 constexpr int kNumTiles = (int)(sizeof(kTiles) / sizeof(kTiles[0]));
 
 static int g_tile_override = -1;  // test hook: force one tile configuration
@@ -80,7 +82,11 @@ static int pick_tile(int m, int n, int k, int mode, int cus, bool packed = false
   // (measured on MI355X: C1 77 -> 68 us, C2 138 -> 106 us; C1 / C2 ffn_out has 32 / 4 tiles of
   // K = 1024 at 64 x 64, 10-11 us, each CU limited by the bytes it keeps in flight).
   if (2 * tiles(4) <= cus) return 5;
-  return 4;  // 64x64: every N that is a multiple of 64
+  // 64x64: every N that is a multiple of 64.  About one tile per CU, so as above a long K wants the stages the
+  // register path keeps in flight (measured on MI355X, direct copies -> registers: 1000 x 1024 x 4096 32.3 -> 19.2 us,
+  // 700 x 1024 x 2048 16.5 -> 9.7, 1500 x 768 x 1536 14.3 -> 12.0, 768 x 1024 x 768 6.4 -> 6.0; K = 512 equal, and
+  // at K = 768 with more tiles than CUs 396 x 3072 x 768 7.5 -> 7.7).
+  return k >= 1024 || (k >= 768 && tiles(4) <= cus) ? 11 : 4;
 }
 
 int device_cus() {
