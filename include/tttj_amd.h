@@ -224,6 +224,12 @@ int tt_forward_packs_rows(int batch, int seq, int d_model, int num_heads, int ff
  * automatic choice.  Process wide, not thread-safe.  No counterpart in the reference. */
 int tt_forward_packing_override(int enable);
 
+/* tt_attention_fwd (prescaled == 0) or tt_attention_fwd_prescaled with a mask whose summary the kernel's
+ * blocks make themselves, so that no tt_mask_info launch precedes it; seq <= 4096. */
+int tt_attention_masked_fwd(const void* q, const void* k, const void* vt, const uint8_t* mask,
+                            void* ctx, int batch, int seq, int heads, int head_dim, int causal,
+                            int prescaled, void* stream);
+
 /* tt_attention_fwd with q already multiplied by hd^-1/2 log2(e) and rounded to fp16 once -- the
  * form the forward's QKV projection writes (tt_stage_offsets) and its attention launches read:
  * ctx = softmax_2(q k^T) v with the same masks.  Replaces the same reference functions as

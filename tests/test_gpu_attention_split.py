@@ -9,7 +9,7 @@ for unit-variance inputs at head_dim 128; together below 5e-3 of what is summed.
 import pytest
 import torch
 
-from tttj_2026_amd import ops
+from tttj_2026_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +48,26 @@ def test_split_attention(hd, causal, mask_kind, s):
         ref[~mask] = 0
         assert not y.view(torch.int16)[~mask].any()
     assert bool(((y.double() - ref).abs() <= 5e-3 * mag + 1e-6).all())
+
+
+@pytest.mark.parametrize("hd", [8, 16, 32, 64, 128, 256])
+@pytest.mark.parametrize("s", [1, 77, 1024, 1500])
+def test_own_mask_summary(hd, s):
+    """A masked call whose blocks summarise the mask themselves equals the call with tt_mask_info's summary bit
+    for bit (16-byte and byte-wise scans, empty, prefix and scattered masks)."""
+    b, h = 4, 1
+    g = torch.Generator().manual_seed(s)
+    q, k = (torch.randn(b, h, s, hd, generator=g).half().cuda() for _ in range(2))
+    vt = torch.randn(b, h, hd, (s + 63) // 64 * 64, generator=g).half().cuda()
+    mask = torch.rand(b, s, generator=g) > 0.4
+    mask[1] = torch.arange(s) < (s + 1) // 2
+    mask[2] = False
+    mask[3] = True
+    mask = mask.cuda()
+    y = ops.attention(q, k, vt, mask, True)
+    info = ops.mask_info(mask, b, s, q.device)
+    z = torch.full_like(y, float("nan"))
+    rc = _lib.load().tt_attention_fwd(q.data_ptr(), k.data_ptr(), vt.data_ptr(), mask.data_ptr(), info.data_ptr(),
+                                      z.data_ptr(), b, s, h, hd, 1, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "tt_attention_fwd")
+    assert torch.equal(y, z)

@@ -48,6 +48,7 @@ SIGNATURES = {
     "tt_pack_derived": (_I, [_P, _I, _I, _I, _P]),
     "tt_mask_info": (_I, [_P, _P, _I, _I, _P]),
     "tt_attention_fwd": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
+    "tt_attention_masked_fwd": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P]),
     "tt_attention_fwd_prescaled": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     "tt_transformer_fwd": (_I, [_P, _P, _P, _P, _P, _I64, _I, _I, _I, _I, _I, _I, _I, _I, _P]),
     "tt_noalloc_scratch_bytes": (_I, [ctypes.POINTER(_I64)]),

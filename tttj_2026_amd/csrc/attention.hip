@@ -68,11 +68,12 @@ float attention_q_scale(int head_dim) {
 
 int launch_attention(const half* q, const half* k, const half* vt, const uint8_t* mask,
                      const int32_t* info, half* ctx, int batch, int seq, int heads, int head_dim,
-                     int causal, hipStream_t stream, bool q_prescaled, const int* out_row) {
+                     int causal, hipStream_t stream, bool q_prescaled, const int* out_row,
+                     bool summarise) {
   TT_REQUIRE(batch > 0 && seq > 0 && heads > 0, "attention: bad shape");
   int rc = attention_head_dim_supported(head_dim);
   if (rc != TT_OK) return rc;
-  TT_REQUIRE(mask == nullptr || info != nullptr, "attention: a mask needs its mask_info");
+  TT_REQUIRE(mask == nullptr || info != nullptr || summarise, "attention: a mask needs its mask_info");
   const AttnArgs args{q, k, vt, mask, ctx, batch, seq, heads, attention_q_scale(head_dim),
                       q_prescaled ? 1 : 0, out_row};
   if (head_dim <= 16) return launch_attention_small(args, info, head_dim, causal, stream);
@@ -100,6 +101,17 @@ extern "C" int tt_attention_fwd(const void* q, const void* k, const void* vt, co
   return tt::launch_attention((const tt::half*)q, (const tt::half*)k, (const tt::half*)vt, mask,
                               info, (tt::half*)ctx, batch, seq, heads, head_dim, causal,
                               (hipStream_t)stream);
+}
+
+extern "C" int tt_attention_masked_fwd(const void* q, const void* k, const void* vt, const uint8_t* mask,
+                                       void* ctx, int batch, int seq, int heads, int head_dim, int causal,
+                                       int prescaled, void* stream) {
+  TT_REQUIRE(q && k && vt && ctx && mask, "attention_masked: null pointer");
+  TT_REQUIRE(seq <= tt::kAttentionSummariseMaxSeq, "attention_masked: sequence of %d > %d (use mask_info)", seq,
+             tt::kAttentionSummariseMaxSeq);
+  return tt::launch_attention((const tt::half*)q, (const tt::half*)k, (const tt::half*)vt, mask, nullptr,
+                              (tt::half*)ctx, batch, seq, heads, head_dim, causal, (hipStream_t)stream,
+                              prescaled != 0, nullptr, true);
 }
 
 extern "C" int tt_attention_fwd_prescaled(const void* q, const void* k, const void* vt,

@@ -60,6 +60,8 @@ __global__ __launch_bounds__(256) void attention_small_kernel(AttnArgs a,
   if (info != nullptr) {
     kv_end = info[b];
     prefix = info[a.B + b] != 0;
+  } else if (a.mask != nullptr) {
+    block_mask_summary<4>(a.mask + (size_t)b * S, S, kv_end, prefix);
   }
   const bool keymask = a.mask != nullptr && !prefix;
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;

@@ -231,6 +231,34 @@ __device__ __forceinline__ float2 combine_row_stats(const float2* part, int slot
   return make_float2(mean, rsqrtf(m2 / (float)K + 1e-5f));
 }
 
+// Last valid position and valid count among mask bytes [0, n) of one sequence, over the lanes
+// i = idx, idx + stride, ...: 16 bytes per lane and step when the row is 16-byte aligned (one
+// load round for n <= 16 stride), bytes otherwise.
+__device__ __forceinline__ void scan_mask(const uint8_t* __restrict__ m, int n, int idx, int stride,
+                                          int& last, int& cnt) {
+  last = -1;
+  cnt = 0;
+  if ((n & 15) == 0 && ((uintptr_t)m & 15) == 0) {
+    for (int c = idx; c < n / 16; c += stride) {
+      const u32x4 w = *(const u32x4*)(m + 16 * c);
+#pragma unroll
+      for (int x = 0; x < 16; ++x) {
+        if ((w[x >> 2] >> (8 * (x & 3))) & 0xFFu) {
+          last = 16 * c + x;
+          ++cnt;
+        }
+      }
+    }
+  } else {
+    for (int s = idx; s < n; s += stride) {
+      if (m[s] != 0) {
+        last = s;
+        ++cnt;
+      }
+    }
+  }
+}
+
 __device__ __forceinline__ float gelu_erf(float v) {
   // Exact-erf GELU, F.gelu(approximate="none"): v * Phi(v), Phi(v) = erfc(-v / sqrt 2) / 2.
   // With z = |v| / sqrt 2, erfc(z) = t * exp(-z^2 + P(t)), t = 1 / (1 + z/2) and P a degree-6

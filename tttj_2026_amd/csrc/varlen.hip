@@ -152,34 +152,6 @@ __global__ __launch_bounds__(256) void varlen_vt_clear_kernel(const uint8_t* __r
 // K rows and V^T entries below its last key tile (as varlen_map_kernel / varlen_vt_clear_kernel).
 constexpr int kPrepSplit = 16;
 
-// Last valid position and valid count among mask bytes [0, n) of one sequence, over the lanes
-// i = idx, idx + stride, ...: 16 bytes per lane and step when the row is 16-byte aligned (one
-// load round for n <= 16 stride), bytes otherwise.
-__device__ __forceinline__ void scan_mask(const uint8_t* __restrict__ m, int n, int idx, int stride,
-                                          int& last, int& cnt) {
-  last = -1;
-  cnt = 0;
-  if ((n & 15) == 0 && ((uintptr_t)m & 15) == 0) {
-    for (int c = idx; c < n / 16; c += stride) {
-      const u32x4 w = *(const u32x4*)(m + 16 * c);
-#pragma unroll
-      for (int x = 0; x < 16; ++x) {
-        if ((w[x >> 2] >> (8 * (x & 3))) & 0xFFu) {
-          last = 16 * c + x;
-          ++cnt;
-        }
-      }
-    }
-  } else {
-    for (int s = idx; s < n; s += stride) {
-      if (m[s] != 0) {
-        last = s;
-        ++cnt;
-      }
-    }
-  }
-}
-
 // kv_end (1 + last valid position), valid count and prefix flag of a sequence's mask, reduced
 // over the block (every thread gets them).
 __device__ __forceinline__ void seq_summary(const uint8_t* __restrict__ mj, int S, int& kv_end,

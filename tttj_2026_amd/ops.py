@@ -14,6 +14,10 @@ import torch
 from . import _lib
 
 
+# Longest sequence whose mask the attention kernels summarise themselves (tt_attention_masked_fwd).
+ATTENTION_SUMMARISE_MAX_SEQ = 4096
+
+
 def _stream(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
@@ -125,7 +129,6 @@ def attention(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor, mask: Optional
         if not t.is_contiguous() or t.dtype != torch.float16:
             raise ValueError(f"{name} must be contiguous fp16")
     mask = _mask(mask, b * s)
-    info = mask_info(mask, b, s, q.device) if mask is not None else None
     if out is None:
         ctx = torch.empty(b, s, h * hd, dtype=torch.float16, device=q.device)
     elif (out.shape != (b, s, h * hd) or out.dtype != torch.float16 or not out.is_contiguous()
@@ -133,6 +136,13 @@ def attention(q: torch.Tensor, k: torch.Tensor, vt: torch.Tensor, mask: Optional
         raise ValueError("out must be a contiguous fp16 [B,S,H*hd] tensor on q's device")
     else:
         ctx = out
+    if mask is not None and s <= ATTENTION_SUMMARISE_MAX_SEQ:
+        rc = _lib.load().tt_attention_masked_fwd(
+            q.data_ptr(), k.data_ptr(), vt.data_ptr(), mask.data_ptr(), ctx.data_ptr(), b, s, h, hd,
+            int(causal), int(prescaled), _stream(q))
+        _lib.check(rc, "tt_attention_masked_fwd")
+        return ctx
+    info = mask_info(mask, b, s, q.device) if mask is not None else None
     fn = _lib.load().tt_attention_fwd_prescaled if prescaled else _lib.load().tt_attention_fwd
     rc = fn(q.data_ptr(), k.data_ptr(), vt.data_ptr(), _ptr(mask), _ptr(info), ctx.data_ptr(), b,
             s, h, hd, int(causal), _stream(q))
