@@ -66,3 +66,24 @@ def test_ragged_qkv(b, s, d, h):
     for got, want in ((q, ref[:, :, 0].permute(0, 2, 1, 3)), (k, ref[:, :, 1].permute(0, 2, 1, 3)),
                       (vt[..., :s], ref[:, :, 2].permute(0, 2, 3, 1))):
         _close(got, want, want)
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("b,s,d,h", [(2, 33, 40, 10), (9, 520, 40, 10), (5, 333, 96, 8), (9, 512, 480, 40),
+                                     (4, 520, 192, 16), (8, 1024, 192, 16), (16, 1024, 256, 64)])
+def test_qkv_heads_off_eight(b, s, d, h, masked):
+    """Head widths that are a multiple of 4 but not of 8 (4, 12), at row counts and widths of every tile;
+    with a mask, whole tiles of padded rows among them."""
+    x, w, bias = _rand((b, s, d), 1), _rand((3 * d, d), 2, 1 / math.sqrt(d)), _rand((3 * d,), 3, 0.5)
+    valid = None
+    if masked:
+        valid = torch.rand(b, s, generator=torch.Generator().manual_seed(6)) > 0.3
+        valid[1] = False
+    q, k, vt = ops.qkv_projection(x, w, bias, h, None if valid is None else valid.cuda())
+    ref = x.cpu().double().reshape(-1, d) @ w.cpu().double().t() + bias.cpu().double()
+    if masked:
+        ref[~valid.reshape(-1)] = 0
+    ref = ref.reshape(b, s, 3, h, d // h)
+    for got, want in ((q, ref[:, :, 0].permute(0, 2, 1, 3)), (k, ref[:, :, 1].permute(0, 2, 1, 3)),
+                      (vt[..., :s], ref[:, :, 2].permute(0, 2, 3, 1))):
+        _close(got, want, want)

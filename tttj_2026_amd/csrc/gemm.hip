@@ -158,10 +158,13 @@ int launch_linear(const half* x, const half* w, int m, int n, int k, const EpiAr
                "linear(qkv): inconsistent shape m=%d n=%d batch=%d seq=%d heads=%d hd=%d", m, n,
                ep.batch, ep.seq, ep.heads, ep.head_dim);
   }
+  // Heads of 4, 12, 20, ... features run on the narrow tiles at every size: their epilogue stores 4 features
+  // at a time, that of the wider tiles 8 of one head.
+  const bool narrow = (ep.mode == TT_EPI_QKV && ep.head_dim % 8 != 0) || linear_is_narrow(m, n, k, ep.mode);
   if (ep.ln_part != nullptr) {
     TT_REQUIRE(ep.mode == TT_EPI_QKV || ep.mode == TT_EPI_BIAS_GELU || ep.mode == TT_EPI_BIAS,
                "linear: a folded LayerNorm needs a bias / GELU / QKV epilogue");
-    TT_REQUIRE(linear_is_narrow(m, n, k, ep.mode),
+    TT_REQUIRE(narrow,
                "linear: a folded LayerNorm runs on the narrow kernels only (m=%d n=%d)", m, n);
     TT_REQUIRE(ep.ln_colsum != nullptr && ep.ln_bias != nullptr && ep.ln_slots > 0 &&
                    k % ep.ln_slots == 0 && ep.ln_stride >= ep.ln_slots,
@@ -174,12 +177,12 @@ int launch_linear(const half* x, const half* w, int m, int n, int k, const EpiAr
     TT_REQUIRE(ep.ln_stride >= n / linear_stats_width(m, n, k, ep.mode),
                "linear: statistics row stride %d < %d slots", ep.ln_stride,
                n / linear_stats_width(m, n, k, ep.mode));
-    TT_REQUIRE(!is_ragged(n, k) || (n % kNarrow == 0 && linear_is_narrow(m, n, k, ep.mode)),
+    TT_REQUIRE(!is_ragged(n, k) || (n % kNarrow == 0 && narrow),
                "linear: row statistics of a ragged shape need the narrow kernel and N %% 32 == 0 "
                "(m=%d n=%d k=%d)", m, n, k);
   }
   if (ep.m_dev != nullptr || ep.rowmap != nullptr) {
-    TT_REQUIRE(!linear_is_narrow(m, n, k, ep.mode),
+    TT_REQUIRE(!narrow,
                "linear: packed variable-length rows run on the MFMA tiles only (m=%d n=%d k=%d)", m,
                n, k);
     TT_REQUIRE(ep.ln_part == nullptr && ep.part_out == nullptr,
@@ -189,9 +192,10 @@ int launch_linear(const half* x, const half* w, int m, int n, int k, const EpiAr
   }
   if (m == 0) return TT_OK;
   if (is_ragged(n, k))
-    return run_ragged(pick_ragged(m, n, ep.mode, device_cus()), x, w, m, n, k, ep, stream);
+    return run_ragged(narrow ? RaggedTile::kNarrow : pick_ragged(m, n, ep.mode, device_cus()), x, w, m, n, k, ep,
+                      stream);
+  if (narrow) return run_narrow(ep.mode, x, w, m, n, k, ep, stream);
   const int tile = pick_tile(m, n, k, ep.mode, device_cus(), ep.m_dev != nullptr);
-  if (tile == 5) return run_narrow(ep.mode, x, w, m, n, k, ep, stream);
   switch (ep.mode) {
     case TT_EPI_BIAS: return run_mode<TT_EPI_BIAS>(tile, x, w, m, n, k, ep, stream);
     case TT_EPI_BIAS_GELU: return run_mode<TT_EPI_BIAS_GELU>(tile, x, w, m, n, k, ep, stream);
