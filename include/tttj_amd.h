@@ -200,7 +200,7 @@ int tt_mask_info(const uint8_t* mask, int32_t* info, int batch, int seq, void* s
 /* Flash attention over the TT_EPI_QKV layout: q, k [B,H,S,hd], vt [B,H,hd,Sp] -> ctx [B,S,H*hd]
  * token-major.  softmax(q k^T * hd^-0.5) with keys masked when (causal && key > query) or
  * mask[b,key] == 0; padded query rows are written as +0.0.  hd in {8, 16, 32, 64, 128, 256}
- * (8 / 16 on the vector ALUs with fp32 probabilities, the others on MFMA).  `info` is the
+ * (8 / 16 with probabilities of 22 bits, the others of fp16's 11).  `info` is the
  * tt_mask_info output for the same mask (may be NULL only if mask is NULL).  Replaces
  * _attention_mxhd (kernels/fused_megakernel.py:544-790) and packed_causal_attention
  * (kernels/case8_attention.py:48-206), and BaselineSelfAttention's score/softmax/PV

@@ -9,9 +9,15 @@
 //   O^T += V^T P^T  v_mfma_f32_16x16x32_f16 over 32 keys: the B operand of lane l is its own 4 + 4
 //                   probabilities of two key tiles, so the A operand takes V^T at those same keys and
 //                   no value crosses lanes.
-// Probabilities keep fp32 precision: p = hi + lo, two fp16 values in two MFMAs, scaled by 2^7 (in the
-// exponent; it cancels in the division by the row sum) so that lo's fp16 granularity is 2^-31 of the
-// largest p and hi still fits after the 2^8 growth the reference max allows; row sums add fp32 values.
+// Probabilities enter as p = hi + lo, two fp16 values in two MFMAs: 22 of fp32's 24 bits (hi is p cut to 11
+// bits, lo the rest), scaled by 2^7 (in the exponent; it cancels in the division by the row sum) so that lo's
+// fp16 granularity is 2^-31 of the largest p and hi still fits after the 2^8 growth the reference max allows;
+// row sums add fp32 values.  The cut is below the rounding of exp2 and of the sums: where P V nearly cancels
+// (values chosen so that the low bits of p are the result) the error against 64 bits is 3.1e-8 of sum p |v|
+// (rms; 1.3e-7 at most), that of fp32 FMAs over single keys, which these MFMAs replaced, 3.4e-8 (1.7e-7).
+// Infinite and NaN values of V, which the split cannot carry (0 inf is NaN), take a second pass with fp32
+// MFMAs (v_mfma_f32_16x16x4_f32: exact products; in the place of the split they made the last shape below
+// 81 -> 124 us).
 // K and V^T fragments are read from global memory straight into registers, the next step's before this
 // one's arithmetic (a head's K and V^T are 16-32 bytes per key and stay in the L1 / L2), so there is no
 // LDS and no barrier.
@@ -223,6 +229,57 @@ __global__ __launch_bounds__(256) void attention_small_kernel(AttnArgs a,
     vf[0] = vn[0];
     vf[1] = vn[1];
     mcur = mnext;
+  }
+
+  // An infinite or NaN value of V leaves no finite output in its feature, whatever the weight: 0 inf and
+  // inf - inf (lo's sign is not hi's) are NaN.  Such a wave starts over with fp32 products, 16 keys at a
+  // time, each key tile only for the query tiles that may attend it.
+  bool odd = false;
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) odd |= !(fabsf(o[t][e]) < INFINITY);
+  if (__builtin_amdgcn_ballot_w64(odd) != 0) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      o[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+      l_run[t] = 0.f;
+      float m = -INFINITY;
+      const int end = CAUSAL ? min(kv_end, qw + 16 * t + 16) : kv_end;
+#pragma unroll 1
+      for (int k0 = 0; k0 < end; k0 += 16) {
+        half4 kk = hzero, vv = hzero;
+        if (klane) kk = *(const half4*)(Kbh + (size_t)min(k0 + col, S - 1) * HD + 4 * g);
+        if (col < HD) vv = *(const half4*)(Vbh + (size_t)col * ldv + k0 + 4 * g);
+        const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+        floatx4 s = __builtin_amdgcn_mfma_f32_16x16x16f16(kk, qf[t], zero, 0, 0, 0);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int key = k0 + 4 * g + j;
+          const bool ok = key < lim[t] && (!keymask || mask[(size_t)b * S + min(key, S - 1)] != 0);
+          s[j] = ok ? (a.q_prescaled ? s[j] : s[j] * a.scale_log2) : -INFINITY;
+          mx = fmaxf(mx, s[j]);
+        }
+        const float m_new = fmaxf(m, quad_rows_max(mx));
+        const bool none = m_new == -INFINITY;  // no allowed key so far
+        const float corr = none ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
+        m = m_new;
+        floatx4 acc;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = o[t][e] *= corr;
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float p = __builtin_amdgcn_exp2f(s[j] - (none ? 0.f : m_new));
+          sum += p;
+          const float v = k0 + 4 * g + j < S ? (float)vv[j] : 0.f;
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(v, p, acc, 0, 0, 0);
+        }
+        l_run[t] = l_run[t] * corr + sum;
+        if (!(none && quad_rows_sum(sum) == 0.f)) o[t] = acc;  // (before the first allowed key: nothing)
+      }
+    }
   }
 
 #pragma unroll
