@@ -288,6 +288,8 @@ def test_stage_offsets():
     assert q == 2 * T * D * 2 and c == -1 and h == q + (2 * T * D + B * D * S) * 2
     q, c, h = _lib.stage_offsets(4, 128, 256, 4, 1024, 2, _lib.PLAN_LAYERWISE)  # folded LN
     assert c == 512 * 256 * 2 and q == 2 * c
+    q, c, h = _lib.stage_offsets(1, 16, 40, 5, 80, 3, _lib.PLAN_LAYERWISE)  # folded, width off the 32 grid
+    assert c >= 0
     q, c, h = _lib.stage_offsets(2, 100, 128, 4, 512, 2, _lib.PLAN_FUSED_LN)
     assert c >= 0
     n = _lib.workspace_bytes(1, 64, 256, 8, 1024, 2, _lib.PLAN_MEGAKERNEL)

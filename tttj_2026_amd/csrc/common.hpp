@@ -147,11 +147,13 @@ __device__ __forceinline__ float seg_sum(float v) {
 
 __device__ __forceinline__ float wave_sum(float v) { return seg_sum<64>(v); }
 
-// Sum over aligned groups of G lanes for G in {4, 8, 16, 32, 64} (quad_perm for 4).
+// Sum over aligned groups of G lanes for G in {2, 4, 8, 16, 32, 64} (quad_perm for 2 and 4).
 template <int G>
 __device__ __forceinline__ float group_sum(float v) {
   if constexpr (G == 1) {
     return v;
+  } else if constexpr (G == 2) {
+    return v + dpp_mov<0xB1>(v);  // quad_perm [1,0,3,2]
   } else if constexpr (G == 4) {
     v += dpp_mov<0xB1>(v);  // quad_perm [1,0,3,2]
     v += dpp_mov<0x4E>(v);  // quad_perm [2,3,0,1]

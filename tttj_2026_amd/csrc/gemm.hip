@@ -131,7 +131,8 @@ bool linear_is_narrow(int m, int n, int k, int mode) {
 }
 
 int linear_stats_width(int m, int n, int k, int mode) {
-  if (is_ragged(n, k)) return kNarrow;         // the ragged tiles write none (launch_linear)
+  // the narrow ragged kernel (epilogue4); the wider ragged tiles write none (launch_linear)
+  if (is_ragged(n, k)) return n % kNarrow == 0 ? kNarrow : 8;
   const int tile = pick_tile(m, n, k, mode, device_cus());
   if (tile == 5) return kNarrow;               // gemm_narrow_kernel: 8 threads per 32 columns
   return kTiles[tile].bn / 2;                  // MFMA tiles: the column range of one wave
@@ -177,9 +178,8 @@ int launch_linear(const half* x, const half* w, int m, int n, int k, const EpiAr
     TT_REQUIRE(ep.ln_stride >= n / linear_stats_width(m, n, k, ep.mode),
                "linear: statistics row stride %d < %d slots", ep.ln_stride,
                n / linear_stats_width(m, n, k, ep.mode));
-    TT_REQUIRE(!is_ragged(n, k) || (n % kNarrow == 0 && narrow),
-               "linear: row statistics of a ragged shape need the narrow kernel and N %% 32 == 0 "
-               "(m=%d n=%d k=%d)", m, n, k);
+    TT_REQUIRE(!is_ragged(n, k) || (narrow && ep.ldy == n),
+               "linear: row statistics of a ragged shape need the narrow kernel (m=%d n=%d k=%d)", m, n, k);
   }
   if (ep.m_dev != nullptr || ep.rowmap != nullptr) {
     TT_REQUIRE(!narrow,

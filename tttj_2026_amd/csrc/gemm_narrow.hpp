@@ -9,9 +9,10 @@
 namespace tt {
 
 // Epilogue of 4 consecutive outputs n .. n + 3 of row m from their fp32 sums (the semantics of
-// gemm_kernel's epilogue, element by element), for the small-shape and narrow-tile kernels.
+// gemm_kernel's epilogue, element by element).
 // G lanes (aligned) share a row and hold consecutive 4-column groups of it: with ep.part_out,
-// they write the partial statistics slot of their 4 G columns; with ep.ln_part, K is the row
+// they write the partial statistics slot of their 4 G columns, or, in a matrix whose width 4 G does not
+// divide, pairs of lanes those of 8 columns (slots are of one width); with ep.ln_part, K is the row
 // length of the folded LayerNorm.
 // Folded-LayerNorm inputs of one thread's 4 outputs, loaded before the GEMM's K loop so their
 // latency overlaps it: the row's (mean, rstd) and the 4 columns' c and b'.
@@ -79,8 +80,14 @@ __device__ __forceinline__ void epilogue4(const EpiArgs& ep, int m, int n, const
         float f[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) f[e] = (float)hv[e];
-        const float2 st = slot_stats<G, 4>(f);
-        if ((threadIdx.x & (G - 1)) == 0) ep.part_out[(size_t)m * ep.ln_stride + n / (4 * G)] = st;
+        float2* const part = ep.part_out + (size_t)m * ep.ln_stride;
+        if (ep.ldy % (4 * G) != 0) {
+          const float2 st = slot_stats<2, 4>(f);
+          if ((threadIdx.x & 1) == 0) part[n / 8] = st;
+        } else {
+          const float2 st = slot_stats<G, 4>(f);
+          if ((threadIdx.x & (G - 1)) == 0) part[n / (4 * G)] = st;
+        }
       }
     } else if (!keep) {
       hv = half4{(half)0.f, (half)0.f, (half)0.f, (half)0.f};
