@@ -47,7 +47,10 @@ extern "C" {
 #define TT_EPI_MASKED_RESID 3
 #define TT_EPI_QKV 4
 
-/* Library version string and the offload architecture it was built for. */
+/* Library version string and the offload architecture it was built for.  0.3: for narrow models (see
+ * tt_weight_layout) the packed weights are longer than 0.2's and every forward but the megakernel's reads the
+ * region that tt_pack_derived fills behind the final norm.  Weights packed by 0.2 must be packed again: the
+ * forward is given no size and would read past their end. */
 const char* tt_version(void);
 
 /* Description of the last failure on the calling thread ("" if none). */

@@ -36,6 +36,12 @@ def test_library_exports_every_declared_symbol():
 def test_version_and_error_channel():
     lib = _lib.load()
     assert b"gfx950" in lib.tt_version()
+    # the version of the packed layout: 0.3 holds a region behind the final norm (two vectors of d_model rounded
+    # up to 64) for narrow models, and only for those
+    assert lib.tt_version().split()[1] == b"0.3"
+    for d, f, extra in ((128, 512, 4 * 128 * 128 + 2 * 128 * 512), (256, 512, 0), (128, 1056, 0), (40, 80, 0)):
+        _, _, final, total = _lib.weight_layout(d, f, 3)
+        assert total == final + 2 * ((d + 63) // 64 * 64) + 3 * extra
     rc = lib.tt_weight_layout(0, 1, 1, None, None, None, None)
     assert rc == _lib.TT_ERR_INVALID
     assert "bad shape" in _lib.last_error()

@@ -160,7 +160,7 @@ using namespace tt;
 
 // 0.2: 18 segments per layer in the packed weights (tt_pack_derived fills 12-17; the folded
 // LayerNorm and megakernel paths read them), packed variable-length rows for masked batches.
-extern "C" const char* tt_version(void) { return "tttj_amd 0.2 gfx950"; }
+extern "C" const char* tt_version(void) { return "tttj_amd 0.3 gfx950"; }
 
 extern "C" const char* tt_last_error_string(void) { return g_last_error.c_str(); }
 
