@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from oracle import transformer_oracle as O
-from tttj_2026_amd import PLAN_LAYERWISE, make_optimized_transformer
+from tttj_2026_amd import PLAN_LAYERWISE, _lib, make_optimized_transformer
 from tttj_2026_amd.configs import build_model, make_inputs
 from tttj_2026_amd.model import TransformerConfig
 
@@ -54,3 +54,18 @@ def test_row_chain(device, b, s, d, h, f, layers, causal, mask_kind):
                                                           None if mask is None else mask[idx], h, causal),
                             None if mask is None else mask[idx])
     assert res["passed"], res
+
+
+def test_short_packed_weights_are_refused(device):
+    """Weights without the region that the row chain reads (as the layout was before it had one)."""
+    cfg = TransformerConfig(2, 40, 64, 2, 96, 2, False)
+    opt = make_optimized_transformer(build_model(cfg, seed=1).half().to(device))
+    x16, _ = make_inputs(cfg, False, 2)
+    with torch.inference_mode():
+        want = opt(x16.to(device)).clone()
+        full, (_, _, final, _) = opt.packed_weights, _lib.weight_layout(64, 96, 2)
+        opt.packed_weights = full[:final + 2 * 64].clone()
+        with pytest.raises(ValueError, match="packed weights"):
+            opt(x16.to(device))
+        opt.packed_weights = full
+        assert torch.equal(opt(x16.to(device)), want)

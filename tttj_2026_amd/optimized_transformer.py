@@ -171,11 +171,13 @@ class OptimizedTransformer(nn.Module):
         self.last_workspace: Optional[torch.Tensor] = None
         self.last_mask: Optional[torch.Tensor] = None
         self._pinned = set()  # megakernel workspaces a captured graph holds
+        self._weight_elems = 0  # of the layout, set by prepare
 
     def prepare(self) -> None:
         check_supported(self.config)
         lib = _lib.load()
         self.packed_weights = pack_model_weights(self.parameter_model)
+        self._weight_elems = self.packed_weights.numel()
         self._lib = lib
 
     def _workspace(self, batch: int, seq: int, plan: int, device: torch.device) -> torch.Tensor:
@@ -314,6 +316,9 @@ class OptimizedTransformer(nn.Module):
             raise ValueError("x must be a CUDA float16 tensor")
         if self.packed_weights.device != x.device or self.packed_weights.dtype != torch.float16:
             raise ValueError("packed weights and input must be fp16 on the same device")
+        if self.packed_weights.numel() < self._weight_elems:  # the library is given no size
+            raise ValueError(f"packed weights of {self.packed_weights.numel()} elements, the layout has "
+                             f"{self._weight_elems} (packed by another version?)")
         batch, seq, _ = x.shape
         x = x.contiguous()
         mask_ptr = None
