@@ -228,7 +228,8 @@ int tt_forward_packs_rows(int batch, int seq, int d_model, int num_heads, int ff
 int tt_forward_packing_override(int enable);
 
 /* tt_attention_fwd (prescaled == 0) or tt_attention_fwd_prescaled with a mask whose summary the kernel's
- * blocks make themselves, so that no tt_mask_info launch precedes it; seq <= 4096. */
+ * blocks make themselves, so that no tt_mask_info launch precedes it; seq <= TT_ATTENTION_SUMMARISE_MAX_SEQ. */
+#define TT_ATTENTION_SUMMARISE_MAX_SEQ 4096
 int tt_attention_masked_fwd(const void* q, const void* k, const void* vt, const uint8_t* mask,
                             void* ctx, int batch, int seq, int heads, int head_dim, int causal,
                             int prescaled, void* stream);

@@ -13,37 +13,12 @@ __global__ __launch_bounds__(256) void mask_info_kernel(const uint8_t* __restric
                                                         int32_t* __restrict__ counts, int B,
                                                         int S) {
   const int b = blockIdx.x;
-  int last = -1, count = 0;
-  if (mask == nullptr) {
-    last = S - 1;
-    count = S;
-  } else {
-    for (int s = threadIdx.x; s < S; s += 256)
-      if (mask[(size_t)b * S + s]) {
-        last = s;
-        ++count;
-      }
-  }
-  __shared__ int sl[256], sc[256];
-  sl[threadIdx.x] = last;
-  sc[threadIdx.x] = count;
-  __syncthreads();
-  for (int off = 128; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) {
-      sl[threadIdx.x] = max(sl[threadIdx.x], sl[threadIdx.x + off]);
-      sc[threadIdx.x] += sc[threadIdx.x + off];
-    }
-    __syncthreads();
-  }
+  int end = S, count = S;
+  if (mask != nullptr) block_mask_summary<4>(mask + (size_t)b * S, S, end, count);
   if (threadIdx.x == 0) {
-    if (mask == nullptr) {
-      info[b] = S;
-      info[B + b] = 1;
-    } else {
-      info[b] = sl[0] + 1;
-      info[B + b] = (sc[0] == sl[0] + 1) ? 1 : 0;
-    }
-    if (counts != nullptr) counts[b] = sc[0];
+    info[b] = end;
+    info[B + b] = count == end;
+    if (counts != nullptr) counts[b] = count;
   }
 }
 
@@ -107,8 +82,8 @@ extern "C" int tt_attention_masked_fwd(const void* q, const void* k, const void*
                                        void* ctx, int batch, int seq, int heads, int head_dim, int causal,
                                        int prescaled, void* stream) {
   TT_REQUIRE(q && k && vt && ctx && mask, "attention_masked: null pointer");
-  TT_REQUIRE(seq <= tt::kAttentionSummariseMaxSeq, "attention_masked: sequence of %d > %d (use mask_info)", seq,
-             tt::kAttentionSummariseMaxSeq);
+  TT_REQUIRE(seq <= TT_ATTENTION_SUMMARISE_MAX_SEQ, "attention_masked: sequence of %d > %d (use mask_info)", seq,
+             TT_ATTENTION_SUMMARISE_MAX_SEQ);
   return tt::launch_attention((const tt::half*)q, (const tt::half*)k, (const tt::half*)vt, mask, nullptr,
                               (tt::half*)ctx, batch, seq, heads, head_dim, causal, (hipStream_t)stream,
                               prescaled != 0, nullptr, true);

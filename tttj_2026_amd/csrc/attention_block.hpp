@@ -442,38 +442,12 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, int bh, int q
 constexpr bool attention_ring3_hd(int hd) { return hd <= 64; }
 inline bool attention_ring3(int hd, int seq) { return attention_ring3_hd(hd) && seq >= 2048; }
 
-// Mask summary of one sequence by a block of NW waves, for launches without mask_info's (every block of the
-// sequence then reads its S mask bytes).  Measured on MI355X per call against a mask_info launch before it: 64 x 4
-// heads of 32, S 128 15.5 -> 8.8 us (host-bound with two launches), 4 x 8 of 128, S 1500 40.0 -> 37.7, 2 x 16 of 64,
-// S 4096 109 -> 107; the forwards share one summary between their layers.
-template <int NW>
-__device__ __forceinline__ void block_mask_summary(const uint8_t* m, int S, int& kv_end, bool& prefix) {
-  __shared__ int s_last[NW], s_cnt[NW];
-  int last, cnt;
-  scan_mask(m, S, threadIdx.x, 64 * NW, last, cnt);
-  for (int off = 32; off > 0; off >>= 1) {
-    last = max(last, __shfl_xor(last, off));
-    cnt += __shfl_xor(cnt, off);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    s_last[threadIdx.x >> 6] = last;
-    s_cnt[threadIdx.x >> 6] = cnt;
-  }
-  __syncthreads();
-  last = s_last[0];
-  cnt = s_cnt[0];
-#pragma unroll
-  for (int w = 1; w < NW; ++w) {
-    last = max(last, s_last[w]);
-    cnt += s_cnt[w];
-  }
-  kv_end = __builtin_amdgcn_readfirstlane(last + 1);
-  prefix = __builtin_amdgcn_readfirstlane(cnt) == kv_end;
-}
-
 // Standalone launch: one block per (b, h, 128-query tile).  `info` (or nullptr without a mask)
 // holds kv_end per sequence and whether its valid keys form a prefix (mask_info_kernel); with a mask and
-// no `info` every block makes its sequence's summary itself.
+// no `info` every block makes its sequence's summary itself (every block of a sequence then reads its S mask
+// bytes).  Measured on MI355X per call against a mask_info launch before it: 64 x 4 heads of 32, S 128 15.5 ->
+// 8.8 us (host-bound with two launches), 4 x 8 of 128, S 1500 40.0 -> 37.7, 2 x 16 of 64, S 4096 109 -> 107; the
+// forwards share one summary between their layers.
 template <int HD, bool CAUSAL, bool RING3, int NSPLIT = 1>
 __global__ __launch_bounds__(256 * NSPLIT) void attention_kernel(AttnArgs a, const int32_t* __restrict__ info) {
   // Dynamic LDS: with statically declared tiles the compiler makes the first K-fragment read of
@@ -494,7 +468,9 @@ __global__ __launch_bounds__(256 * NSPLIT) void attention_kernel(AttnArgs a, con
     kv_end = info[b];
     prefix = info[a.B + b] != 0;
   } else if (a.mask != nullptr) {
-    block_mask_summary<4 * NSPLIT>(a.mask + (size_t)b * a.S, a.S, kv_end, prefix);
+    int count;
+    block_mask_summary<4 * NSPLIT>(a.mask + (size_t)b * a.S, a.S, kv_end, count);
+    prefix = count == kv_end;
   }
   // A query tile at or past the last valid key holds only padded rows: they are +0.0 (or, with a
   // packed output map, not stored at all), and the key loop -- whose copies and barriers such a

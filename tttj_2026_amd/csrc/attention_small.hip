@@ -67,7 +67,9 @@ __global__ __launch_bounds__(256) void attention_small_kernel(AttnArgs a,
     kv_end = info[b];
     prefix = info[a.B + b] != 0;
   } else if (a.mask != nullptr) {
-    block_mask_summary<4>(a.mask + (size_t)b * S, S, kv_end, prefix);
+    int count;
+    block_mask_summary<4>(a.mask + (size_t)b * S, S, kv_end, count);
+    prefix = count == kv_end;
   }
   const bool keymask = a.mask != nullptr && !prefix;
   const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;

@@ -261,6 +261,34 @@ __device__ __forceinline__ void scan_mask(const uint8_t* __restrict__ m, int n, 
   }
 }
 
+// Mask summary of one sequence by a block of NW waves (every thread gets it): 1 + the last valid position, and
+// the number of valid tokens, which is the same where they form a prefix.
+template <int NW>
+__device__ __forceinline__ void block_mask_summary(const uint8_t* __restrict__ m, int S, int& kv_end,
+                                                   int& count) {
+  __shared__ int s_last[NW], s_cnt[NW];
+  int last, cnt;
+  scan_mask(m, S, threadIdx.x, 64 * NW, last, cnt);
+  for (int off = 32; off > 0; off >>= 1) {
+    last = max(last, __shfl_xor(last, off));
+    cnt += __shfl_xor(cnt, off);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    s_last[threadIdx.x >> 6] = last;
+    s_cnt[threadIdx.x >> 6] = cnt;
+  }
+  __syncthreads();
+  last = s_last[0];
+  cnt = s_cnt[0];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) {
+    last = max(last, s_last[w]);
+    cnt += s_cnt[w];
+  }
+  kv_end = __builtin_amdgcn_readfirstlane(last + 1);
+  count = __builtin_amdgcn_readfirstlane(cnt);
+}
+
 __device__ __forceinline__ float gelu_erf(float v) {
   // Exact-erf GELU, F.gelu(approximate="none"): v * Phi(v), Phi(v) = erfc(-v / sqrt 2) / 2.
   // With z = |v| / sqrt 2, erfc(z) = t * exp(-z^2 + P(t)), t = 1 / (1 + z/2) and P a degree-6

@@ -91,8 +91,6 @@ int launch_attention(const half* q, const half* k, const half* vt, const uint8_t
                      const int32_t* info, half* ctx, int batch, int seq, int heads, int head_dim,
                      int causal, hipStream_t stream, bool q_prescaled = false,
                      const int* out_row = nullptr, bool summarise = false);
-// Sequence length up to which launch_attention takes a mask without info (`summarise`).
-constexpr int kAttentionSummariseMaxSeq = 4096;
 // hd^-1/2 log2(e): the factor of the scores in the exp2-domain softmax.
 float attention_q_scale(int head_dim);
 int attention_head_dim_supported(int head_dim);

@@ -83,27 +83,9 @@ __global__ __launch_bounds__(kChainThreads, 2) void rowchain_kernel(ChainArgs a)
     // One block per sequence behind them: the mask summary the attention launches read (as
     // mask_info_kernel), beside the row tiles instead of in a launch of its own.
     const int b = blockIdx.x - nblocks;
-    int end = 0, count = 0;
-    for (int s = tid; s < S; s += NT)
-      if (a.valid[(size_t)b * S + s] != 0) {
-        end = s + 1;
-        ++count;
-      }
-    __shared__ int s_end[8], s_count[8];
-    for (int off = 32; off > 0; off >>= 1) {
-      end = max(end, __shfl_xor(end, off));
-      count += __shfl_xor(count, off);
-    }
-    if (lane == 0) {
-      s_end[wave] = end;
-      s_count[wave] = count;
-    }
-    __syncthreads();
+    int end, count;
+    block_mask_summary<kChainThreads / 64>(a.valid + (size_t)b * S, S, end, count);
     if (tid == 0) {
-      for (int w = 1; w < 8; ++w) {
-        end = max(end, s_end[w]);
-        count += s_count[w];
-      }
       a.info[b] = end;
       a.info[a.info_blocks + b] = count == end;
     }

@@ -152,29 +152,6 @@ __global__ __launch_bounds__(256) void varlen_vt_clear_kernel(const uint8_t* __r
 // K rows and V^T entries below its last key tile (as varlen_map_kernel / varlen_vt_clear_kernel).
 constexpr int kPrepSplit = 16;
 
-// kv_end (1 + last valid position), valid count and prefix flag of a sequence's mask, reduced
-// over the block (every thread gets them).
-__device__ __forceinline__ void seq_summary(const uint8_t* __restrict__ mj, int S, int& kv_end,
-                                            int& cnt, bool& prefix) {
-  __shared__ int s_red[2][4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int last, c;
-  scan_mask(mj, S, tid, 256, last, c);
-  for (int off = 32; off > 0; off >>= 1) {
-    last = max(last, __shfl_xor(last, off));
-    c += __shfl_xor(c, off);
-  }
-  if (lane == 0) {
-    s_red[0][wave] = last;
-    s_red[1][wave] = c;
-  }
-  __syncthreads();
-  last = max(max(s_red[0][0], s_red[0][1]), max(s_red[0][2], s_red[0][3]));
-  cnt = s_red[1][0] + s_red[1][1] + s_red[1][2] + s_red[1][3];
-  kv_end = last + 1;
-  prefix = cnt == kv_end;
-}
-
 __global__ __launch_bounds__(256) void varlen_prep_kernel(
     const uint8_t* __restrict__ mask, int32_t* __restrict__ info, int32_t* __restrict__ counts,
     int32_t* __restrict__ n_dev, int32_t* __restrict__ row_tok, int32_t* __restrict__ slot,
@@ -184,8 +161,8 @@ __global__ __launch_bounds__(256) void varlen_prep_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const size_t tok0 = (size_t)b * S;
   int kv_end, cnt;
-  bool prefix;
-  seq_summary(mask + tok0, S, kv_end, cnt, prefix);
+  block_mask_summary<4>(mask + tok0, S, kv_end, cnt);
+  const bool prefix = cnt == kv_end;
   const int ldv = (S + 63) / 64 * 64;
   const int end = min(S, (kv_end + 63) & ~63);  // keys the attention's tiles read
   if (y == 0) {

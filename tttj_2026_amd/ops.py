@@ -14,7 +14,8 @@ import torch
 from . import _lib
 
 
-# Longest sequence whose mask the attention kernels summarise themselves (tt_attention_masked_fwd).
+# Longest sequence whose mask the attention kernels summarise themselves (tt_attention_masked_fwd; the header's
+# TT_ATTENTION_SUMMARISE_MAX_SEQ).
 ATTENTION_SUMMARISE_MAX_SEQ = 4096
 
 
