@@ -37,7 +37,6 @@ namespace tt {
 
 constexpr int kChainFC = 128;  // hidden columns per chunk: 16 per wave
 constexpr int kChainThreads = 512;
-constexpr int kChainBlocks = 256;  // CUs
 
 // LDS: residual stream and LayerNorm output [R][D + 8], two hidden chunks [R][136], and the fp16 vectors
 // bo, norm2 gain / bias, b2, norm1 gain / bias (or the final norm's), bqkv, b1.
@@ -499,7 +498,7 @@ static int run_chain(const ChainArgs& a, hipStream_t stream) {
   if (attr != hipSuccess)
     return fail(TT_ERR_HIP, "hipFuncSetAttribute(rowchain): %s", hipGetErrorString(attr));
   int blocks = (a.T + 16 * RT - 1) / (16 * RT);
-  if (KEEP) blocks = std::min(blocks, kChainBlocks);
+  if (KEEP) blocks = std::min(blocks, device_cus());
   if (!MID) blocks += a.info_blocks;
   hipLaunchKernelGGL((rowchain_kernel<D, RT, MID, KEEP>), dim3(blocks), dim3(kChainThreads),
                      chain_lds_bytes(D, RT, MID ? a.F : 0), stream, a);
@@ -513,7 +512,7 @@ static int run_chain_mid(const ChainArgs& a, bool mid, hipStream_t stream) {
 
 template <int D>
 static int run_chain_d(const ChainArgs& a, bool mid, hipStream_t stream) {
-  const bool many = a.T > 32 * kChainBlocks;
+  const bool many = a.T > 32 * device_cus();
   if constexpr (D <= 128) {
     if (a.F <= kChainFC)
       return many ? run_chain_mid<D, 4, true>(a, mid, stream) : run_chain_mid<D, 2, true>(a, mid, stream);
