@@ -115,7 +115,10 @@ static bool is_ragged(int n, int k) { return k % kBK != 0 || n % 64 != 0; }
 // 15.7 -> 16.8, the worst of ten shapes), 32 x 32 narrow tiles where 64 x 64 would fill at most half the
 // CUs (the rule of the aligned widths), else 64 x 64.  Against the vector-ALU kernel these replaced:
 // 1600 x 480 x 160 (QKV) 58 -> 5 us, 1600 x 640 x 160 91 -> 6 us.
-static RaggedTile pick_ragged(int m, int n, int mode, int cus) {
+// Rows of 2^22 values and more stay on the narrow tiles, which address each row by a pointer: the others mark
+// loads past K by a buffer offset just below 2^31, which has to lie past the tile's 128 rows.
+static RaggedTile pick_ragged(int m, int n, int k, int mode, int cus) {
+  if (k >= 1 << 22) return RaggedTile::kNarrow;
   auto tiles = [&](int bm, int bn) {
     const long cols = mode == TT_EPI_QKV ? 3 * ((n / 3 + bn - 1) / bn) : (n + bn - 1) / bn;
     return (long)((m + bm - 1) / bm) * cols;
@@ -126,7 +129,7 @@ static RaggedTile pick_ragged(int m, int n, int mode, int cus) {
 }
 
 bool linear_is_narrow(int m, int n, int k, int mode) {
-  if (is_ragged(n, k)) return pick_ragged(m, n, mode, device_cus()) == RaggedTile::kNarrow;
+  if (is_ragged(n, k)) return pick_ragged(m, n, k, mode, device_cus()) == RaggedTile::kNarrow;
   return pick_tile(m, n, k, mode, device_cus()) == 5;
 }
 
@@ -192,7 +195,7 @@ int launch_linear(const half* x, const half* w, int m, int n, int k, const EpiAr
   }
   if (m == 0) return TT_OK;
   if (is_ragged(n, k))
-    return run_ragged(narrow ? RaggedTile::kNarrow : pick_ragged(m, n, ep.mode, device_cus()), x, w, m, n, k, ep,
+    return run_ragged(narrow ? RaggedTile::kNarrow : pick_ragged(m, n, k, ep.mode, device_cus()), x, w, m, n, k, ep,
                       stream);
   if (narrow) return run_narrow(ep.mode, x, w, m, n, k, ep, stream);
   const int tile = pick_tile(m, n, k, ep.mode, device_cus(), ep.m_dev != nullptr);
