@@ -52,13 +52,15 @@ __device__ __forceinline__ float quad_rows_sum(float v) {
 
 template <int HD, bool CAUSAL>
 __global__ __launch_bounds__(256) void attention_small_kernel(AttnArgs a,
-                                                              const int32_t* __restrict__ info) {
+                                                              const int32_t* __restrict__ info,
+                                                              unsigned first_block) {
   constexpr float kLazy = 8.0f;  // log2 growth of the row max that moves the reference
   const int S = a.S, H = a.H;
   const int BH = a.B * H;
   const int nqt = (S + kSmallBQ - 1) / kSmallBQ;
-  const int bh = blockIdx.x % BH;
-  int qt = blockIdx.x / BH;
+  const int block = (int)(first_block + blockIdx.x);
+  const int bh = block % BH;
+  int qt = block / BH;
   if (CAUSAL) qt = nqt - 1 - qt;
   const int b = bh / H, h = bh - b * H;
   int kv_end = S;
@@ -311,9 +313,10 @@ int launch_attention_small(const AttnArgs& args, const int32_t* info, int head_d
              head_dim);
   const long blocks = (long)args.B * args.H * ((args.S + kSmallBQ - 1) / kSmallBQ);
   TT_REQUIRE(blocks < (1L << 31), "attention: grid too large");
-  const dim3 grid((unsigned)blocks), block(256);
-#define TT_ATT_SMALL(HD, C) \
-  hipLaunchKernelGGL((attention_small_kernel<HD, C>), grid, block, 0, stream, args, info)
+#define TT_ATT_SMALL(HD, C)                                                                             \
+  launch_in_parts(blocks, 256, [&](unsigned first, unsigned n) {                                        \
+    hipLaunchKernelGGL((attention_small_kernel<HD, C>), dim3(n), dim3(256), 0, stream, args, info, first); \
+  })
   if (head_dim == 8) {
     if (causal) TT_ATT_SMALL(8, true); else TT_ATT_SMALL(8, false);
   } else {

@@ -118,10 +118,12 @@ constexpr size_t narrow_lds_bytes(int nw) { return (size_t)nw * 2 * kNarrowSlice
 template <int MODE, int NW, bool RAG>
 __global__ __launch_bounds__(64 * NW) void gemm_narrow_kernel(const half* __restrict__ X,
                                                               const half* __restrict__ W, int M,
-                                                              int N, int K, EpiArgs ep) {
+                                                              int N, int K, EpiArgs ep,
+                                                              unsigned first_block) {
   extern __shared__ __align__(16) half lds[];
   const int tiles_n = column_tiles<kNarrow, MODE, RAG>(N);
-  const int tm = blockIdx.x / tiles_n, tn = blockIdx.x - tm * tiles_n;
+  const int block = (int)(first_block + blockIdx.x);
+  const int tm = block / tiles_n, tn = block - tm * tiles_n;
   const int m0 = tm * kNarrow;
   int n0 = tn * kNarrow;
   [[maybe_unused]] int n_end = N;
@@ -233,8 +235,10 @@ static int launch_narrow_waves(const half* x, const half* w, int m, int n, int k
     return fail(TT_ERR_HIP, "hipFuncSetAttribute(gemm_narrow): %s", hipGetErrorString(attr));
   const long blocks = (long)((m + kNarrow - 1) / kNarrow) * column_tiles<kNarrow, MODE, RAG>(n);
   TT_REQUIRE(blocks < (1L << 31), "linear: grid too large");
-  hipLaunchKernelGGL((gemm_narrow_kernel<MODE, NW, RAG>), dim3((unsigned)blocks), dim3(64 * NW),
-                     narrow_lds_bytes(NW), stream, x, w, m, n, k, ep);
+  launch_in_parts(blocks, 64 * NW, [&](unsigned first, unsigned part) {
+    hipLaunchKernelGGL((gemm_narrow_kernel<MODE, NW, RAG>), dim3(part), dim3(64 * NW), narrow_lds_bytes(NW),
+                       stream, x, w, m, n, k, ep, first);
+  });
   return launch_status("gemm_narrow_kernel");
 }
 

@@ -38,6 +38,14 @@ struct EpiArgs {
 
 int device_cus();  // compute units of the current device
 
+// A launch may have at most 2^32 - 1 threads.  Larger grids go out in parts: launch(first block, blocks).
+template <class Launch>
+inline void launch_in_parts(long blocks, int threads, Launch launch) {
+  const long most = ((1L << 32) - 1) / threads;
+  for (long first = 0; first < blocks; first += most)
+    launch((unsigned)first, (unsigned)(blocks - first < most ? blocks - first : most));
+}
+
 int launch_layernorm(const half* x, const half* gamma, const half* beta, const uint8_t* valid,
                      half* y, int rows, int d, float eps, hipStream_t stream);
 // LayerNorm over packed variable-length rows: output row r reads input row in_row[r] (r itself
