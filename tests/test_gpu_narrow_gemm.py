@@ -22,3 +22,23 @@ def test_narrow_slices(m, n, k):
     y = ops.linear(x.cuda(), w.cuda(), b.cuda(), "masked_resid", residual=r.cuda()).cpu().double()
     ref = branch + r.double()
     assert bool(((y - ref).abs() <= 2.0 ** -11 * (ref.abs() + branch.abs()) + 2e-4).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 64, 128), (40, 192, 1024), (33, 72, 40), (5, 40, 1032), (4000, 72, 136)])
+@pytest.mark.parametrize("mode", ["bias", "resid_masked"])
+def test_operands_at_any_offset(device, m, n, k, mode):
+    """Contiguous operands that start at any fp16 value of a buffer give what aligned ones give, bit for bit where
+    both run on narrow tiles."""
+    g = torch.Generator().manual_seed(1)
+    at = {name: (torch.randn(*s, generator=g) * c).half().to(device)
+          for name, s, c in (("x", (m, k), 1), ("w", (n, k), k ** -0.5), ("b", (n,), 1), ("r", (m, n), 1))}
+    off = {}
+    for i, (name, t) in enumerate(at.items()):
+        buf = torch.empty(t.numel() + 8, dtype=t.dtype, device=device)
+        off[name] = buf[1 + 2 * i:1 + 2 * i + t.numel()].view(t.shape).copy_(t)
+        assert off[name].is_contiguous() and off[name].data_ptr() % 16 != 0
+    y, want = (ops.linear(t["x"], t["w"], t["b"], mode, residual=t["r"] if mode != "bias" else None) for t in (off, at))
+    if m < 100:
+        assert torch.equal(y, want)
+    else:  # sums of k products in another order
+        assert bool(((y - want).abs().double() <= 2.0 ** -10 * want.abs().double() + 1e-4).all())

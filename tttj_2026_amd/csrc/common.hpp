@@ -18,6 +18,7 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // load + store pair into a memcpy placed at the store, which would delay a prefetch load.
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x4 u32x4_any __attribute__((aligned(2)));  // 16 bytes at any address of a half
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kWave = 64;

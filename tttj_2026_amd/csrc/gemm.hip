@@ -164,7 +164,10 @@ int launch_linear(const half* x, const half* w, int m, int n, int k, const EpiAr
   }
   // Heads of 4, 12, 20, ... features run on the narrow tiles at every size: their epilogue stores 4 features
   // at a time, that of the wider tiles 8 of one head.
-  const bool narrow = (ep.mode == TT_EPI_QKV && ep.head_dim % 8 != 0) || linear_is_narrow(m, n, k, ep.mode);
+  // Ragged shapes with an operand that is not 16-byte aligned run on the narrow tiles too, in their staged form.
+  const bool unaligned = (((uintptr_t)x | (uintptr_t)w) & 15) != 0;
+  const bool narrow = (ep.mode == TT_EPI_QKV && ep.head_dim % 8 != 0) ||
+                      (unaligned && is_ragged(n, k) && ep.m_dev == nullptr) || linear_is_narrow(m, n, k, ep.mode);
   if (ep.ln_part != nullptr) {
     TT_REQUIRE(ep.mode == TT_EPI_QKV || ep.mode == TT_EPI_BIAS_GELU || ep.mode == TT_EPI_BIAS,
                "linear: a folded LayerNorm needs a bias / GELU / QKV epilogue");
@@ -194,6 +197,7 @@ int launch_linear(const half* x, const half* w, int m, int n, int k, const EpiAr
                "linear(qkv): packed rows need both the row count and the row map");
   }
   if (m == 0) return TT_OK;
+  if (narrow && unaligned) return run_ragged(RaggedTile::kNarrowStaged, x, w, m, n, k, ep, stream);
   if (is_ragged(n, k))
     return run_ragged(narrow ? RaggedTile::kNarrow : pick_ragged(m, n, k, ep.mode, device_cus()), x, w, m, n, k, ep,
                       stream);

@@ -111,11 +111,14 @@ __device__ __forceinline__ void epilogue4(const EpiArgs& ep, int m, int n, const
 // RAG: N (for the QKV projection each of its three parts) and K are multiples of 8 only.  A part's last
 // column tile is then partial: W rows past the part are clamped to its last one and their outputs not
 // stored.  8-value chunks at or past K are replaced by zeros when they are read from LDS.
+//
+// STAGED: X or W is not 16-byte aligned.  The copies go through registers, by plain loads, which take any
+// alignment; nothing is documented for the direct copies.
 constexpr int kNarrow = 32;
 constexpr int kNarrowSlice = 2 * kNarrow * kBK;  // halfs: X rows 0 .. 31, W rows 32 .. 63
 constexpr size_t narrow_lds_bytes(int nw) { return (size_t)nw * 2 * kNarrowSlice * sizeof(half); }
 
-template <int MODE, int NW, bool RAG>
+template <int MODE, int NW, bool RAG, bool STAGED = false>
 __global__ __launch_bounds__(64 * NW) void gemm_narrow_kernel(const half* __restrict__ X,
                                                               const half* __restrict__ W, int M,
                                                               int N, int K, EpiArgs ep,
@@ -153,7 +156,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_narrow_kernel(const half* __rest
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
       const int k = s * kBK + col[c & 1];
-      lds_copy16(src[c] + (RAG && k >= K ? 0 : k), ring + slot * kNarrowSlice + c * 512);
+      const half* p = src[c] + (RAG && k >= K ? 0 : k);
+      half* dst = ring + slot * kNarrowSlice + c * 512;
+      if constexpr (STAGED) *(u32x4*)(dst + 8 * lane) = *(const u32x4_any*)p;
+      else lds_copy16(p, dst);
     }
   };
   // slices wave, wave + NW, ...
@@ -222,13 +228,13 @@ __global__ __launch_bounds__(64 * NW) void gemm_narrow_kernel(const half* __rest
 // 8 waves above K = 512 (more than the two slices per wave that 4 waves hold at once).
 static bool narrow_long_k(int k) { return k > 512; }
 
-template <int MODE, int NW, bool RAG>
+template <int MODE, int NW, bool RAG, bool STAGED>
 static int launch_narrow_waves(const half* x, const half* w, int m, int n, int k, const EpiArgs& ep,
                                hipStream_t stream) {
   static std::once_flag once;
   static hipError_t attr = hipSuccess;
   std::call_once(once, [] {
-    attr = hipFuncSetAttribute((const void*)gemm_narrow_kernel<MODE, NW, RAG>,
+    attr = hipFuncSetAttribute((const void*)gemm_narrow_kernel<MODE, NW, RAG, STAGED>,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)narrow_lds_bytes(NW));
   });
   if (attr != hipSuccess)
@@ -236,17 +242,17 @@ static int launch_narrow_waves(const half* x, const half* w, int m, int n, int k
   const long blocks = (long)((m + kNarrow - 1) / kNarrow) * column_tiles<kNarrow, MODE, RAG>(n);
   TT_REQUIRE(blocks < (1L << 31), "linear: grid too large");
   launch_in_parts(blocks, 64 * NW, [&](unsigned first, unsigned part) {
-    hipLaunchKernelGGL((gemm_narrow_kernel<MODE, NW, RAG>), dim3(part), dim3(64 * NW), narrow_lds_bytes(NW),
+    hipLaunchKernelGGL((gemm_narrow_kernel<MODE, NW, RAG, STAGED>), dim3(part), dim3(64 * NW), narrow_lds_bytes(NW),
                        stream, x, w, m, n, k, ep, first);
   });
   return launch_status("gemm_narrow_kernel");
 }
 
-template <int MODE, bool RAG>
+template <int MODE, bool RAG, bool STAGED = false>
 static int launch_narrow_mode(const half* x, const half* w, int m, int n, int k, const EpiArgs& ep,
                               hipStream_t stream) {
-  return narrow_long_k(k) ? launch_narrow_waves<MODE, 8, RAG>(x, w, m, n, k, ep, stream)
-                          : launch_narrow_waves<MODE, 4, RAG>(x, w, m, n, k, ep, stream);
+  return narrow_long_k(k) ? launch_narrow_waves<MODE, 8, RAG, STAGED>(x, w, m, n, k, ep, stream)
+                          : launch_narrow_waves<MODE, 4, RAG, STAGED>(x, w, m, n, k, ep, stream);
 }
 
 }  // namespace tt

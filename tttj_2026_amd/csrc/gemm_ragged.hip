@@ -11,6 +11,7 @@ static int run_ragged_mode(RaggedTile tile, const half* x, const half* w, int m,
   switch (tile) {
     case RaggedTile::k128x128: return run_tile<128, 128, MODE, 1, 4, true>(x, w, m, n, k, ep, stream);
     case RaggedTile::k64x64: return run_tile<64, 64, MODE, 1, 4, true>(x, w, m, n, k, ep, stream);
+    case RaggedTile::kNarrowStaged: return launch_narrow_mode<MODE, true, true>(x, w, m, n, k, ep, stream);
     default: return launch_narrow_mode<MODE, true>(x, w, m, n, k, ep, stream);
   }
 }

@@ -58,8 +58,9 @@ int launch_layernorm_rows(const half* x, const half* gamma, const half* beta, co
 
 int launch_linear(const half* x, const half* w, int m, int n, int k, const EpiArgs& ep,
                   hipStream_t stream);
-// Tiles of the GEMM kernels for ragged widths (gemm_ragged.hip).
-enum class RaggedTile { kNarrow, k64x64, k128x128 };
+// Tiles of the GEMM kernels for ragged widths (gemm_ragged.hip); kNarrowStaged is kNarrow for operands that are
+// not 16-byte aligned.
+enum class RaggedTile { kNarrow, kNarrowStaged, k64x64, k128x128 };
 int run_ragged(RaggedTile tile, const half* x, const half* w, int m, int n, int k, const EpiArgs& ep,
                hipStream_t stream);
 // Columns per partial-statistics slot the GEMM launch_linear would run for this shape writes
