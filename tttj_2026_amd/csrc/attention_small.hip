@@ -51,9 +51,9 @@ __device__ __forceinline__ float quad_rows_sum(float v) {
 }
 
 template <int HD, bool CAUSAL>
-__global__ __launch_bounds__(256) void attention_small_kernel(AttnArgs a,
+__global__ __launch_bounds__(256) void attention_small_kernel(unsigned first_block,
                                                               const int32_t* __restrict__ info,
-                                                              unsigned first_block) {
+                                                              AttnArgs a) {
   constexpr float kLazy = 8.0f;  // log2 growth of the row max that moves the reference
   const int S = a.S, H = a.H;
   const int BH = a.B * H;
@@ -315,7 +315,7 @@ int launch_attention_small(const AttnArgs& args, const int32_t* info, int head_d
   TT_REQUIRE(blocks < (1L << 31), "attention: grid too large");
 #define TT_ATT_SMALL(HD, C)                                                                             \
   launch_in_parts(blocks, 256, [&](unsigned first, unsigned n) {                                        \
-    hipLaunchKernelGGL((attention_small_kernel<HD, C>), dim3(n), dim3(256), 0, stream, args, info, first); \
+    hipLaunchKernelGGL((attention_small_kernel<HD, C>), dim3(n), dim3(256), 0, stream, first, info, args); \
   })
   if (head_dim == 8) {
     if (causal) TT_ATT_SMALL(8, true); else TT_ATT_SMALL(8, false);

@@ -121,8 +121,8 @@ constexpr size_t narrow_lds_bytes(int nw) { return (size_t)nw * 2 * kNarrowSlice
 template <int MODE, int NW, bool RAG, bool STAGED = false>
 __global__ __launch_bounds__(64 * NW) void gemm_narrow_kernel(const half* __restrict__ X,
                                                               const half* __restrict__ W, int M,
-                                                              int N, int K, EpiArgs ep,
-                                                              unsigned first_block) {
+                                                              int N, int K, unsigned first_block,
+                                                              EpiArgs ep) {
   extern __shared__ __align__(16) half lds[];
   const int tiles_n = column_tiles<kNarrow, MODE, RAG>(N);
   const int block = (int)(first_block + blockIdx.x);
@@ -243,7 +243,7 @@ static int launch_narrow_waves(const half* x, const half* w, int m, int n, int k
   TT_REQUIRE(blocks < (1L << 31), "linear: grid too large");
   launch_in_parts(blocks, 64 * NW, [&](unsigned first, unsigned part) {
     hipLaunchKernelGGL((gemm_narrow_kernel<MODE, NW, RAG, STAGED>), dim3(part), dim3(64 * NW), narrow_lds_bytes(NW),
-                       stream, x, w, m, n, k, ep, first);
+                       stream, x, w, m, n, k, first, ep);
   });
   return launch_status("gemm_narrow_kernel");
 }
