@@ -371,12 +371,14 @@ def test_pack_derived_segments(device):
 
 @pytest.mark.parametrize("shape", [(2, 64, 256, 4, 1024, 3, False, False),
                                    (3, 100, 512, 8, 2048, 2, True, True),
-                                   (1, 32, 96, 3, 160, 2, True, False)],
-                         ids=["D256", "D512-masked", "D96-small-kernel"])
+                                   (1, 32, 96, 3, 160, 2, True, False),
+                                   (1, 32, 224, 7, 480, 2, True, False)],
+                         ids=["D256", "D512-masked", "D96-row-chain", "D224-ragged"])
 def test_folded_layernorm_large_input_perturbed_norms(device, shape):
     """The folded LayerNorm (statistics from the producer's partial slots, W' and the epilogue
     correction) at input scale 30 with non-default LayerNorm parameters: the gate still holds,
-    so the single-pass partial statistics and the rstd (acc - mean c) form do not cancel badly."""
+    so the single-pass partial statistics and the rstd (acc - mean c) form do not cancel badly.
+    (D96 runs the row chain, whose LayerNorms are its own.)"""
     b, s, d, h, f, l, causal, masked = shape
     cfg = TransformerConfig(b, s, d, h, f, l, causal)
     model = build_model(cfg, seed=41)
@@ -440,12 +442,16 @@ def test_folded_layernorm_matches_fused_ln_plan(device, name):
 @pytest.mark.parametrize("plan_name,shape", [
     ("megakernel", (2, 64, 256, 8, 1024, True, True)),      # hd 32, causal, padded
     ("megakernel", (1, 64, 256, 4, 1024, False, False)),    # hd 64
-    ("fused_ln", (2, 100, 128, 4, 512, True, True)),
+    ("fused_ln", (2, 100, 128, 4, 512, True, True)),        # narrow model: the row chain in this plan
+    ("fused_ln", (2, 100, 256, 4, 512, True, True)),        # LayerNorms inside the QKV / ffn_in tiles
+    ("fused_ln", (3, 50, 128, 4, 1280, False, True)),       # the same, ffn_dim too wide for the row chain
     ("layerwise", (4, 128, 256, 4, 1024, False, True)),     # LayerNorm folded (narrow tiles)
+    ("layerwise", (2, 33, 72, 9, 144, True, True)),         # folded, ragged widths
     ("layerwise", (2, 256, 512, 8, 2048, True, False)),     # MFMA tiles; LN2 overwrites ctx
     ("layerwise", (4, 512, 512, 16, 2048, True, True)),     # packed variable-length rows
-], ids=["mk-hd32-causal-mask", "mk-hd64", "fusedln-causal-mask", "lw-fold-mask", "lw-mfma-causal",
-        "lw-packed-mask"])
+    ("layerwise", (8, 300, 288, 9, 584, False, True)),      # packed, ragged widths
+], ids=["mk-hd32-causal-mask", "mk-hd64", "chain-causal-mask", "fusedln-d256-causal-mask", "fusedln-f1280-mask",
+        "lw-fold-mask", "lw-fold-ragged-mask", "lw-mfma-causal", "lw-packed-mask", "lw-packed-ragged-mask"])
 def test_captured_stages(device, plan_name, shape):
     """Per-stage parity inside the fused plans (after benchmarks/benchmark_steps_1_2.py:73-117 and
     the CAPTURE slots of kernels/fused_megakernel.py:224-238): the last layer's Q / K / V, attention

@@ -25,7 +25,9 @@ CASES = [
     (3, 200, 256, 4, 512, 2, True, "prefix"),
     (2, 77, 256, 8, 256, 3, False, "nonprefix"),
     (2, 256, 512, 8, 2048, 2, True, "prefix"),     # D = 512: the W ring wraps
-    (5, 33, 128, 4, 128, 1, True, "empty"),
+    (5, 33, 128, 4, 128, 1, True, "empty"),        # narrow: both plans run the row chain
+    (5, 33, 256, 4, 256, 1, True, "empty"),
+    (4, 60, 128, 4, 1280, 2, False, "empty"),      # ffn_dim too wide for the row chain
 ]
 
 
@@ -76,6 +78,30 @@ def test_fused_ln_parity(device, case):
     assert res["passed"], res
     assert torch.equal(y1, y2)
     assert (y1.float() - ylw.float()).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("b,s,d,h,f,causal,kind", [(3, 66, 128, 4, 1280, True, "empty"),
+                                                   (2, 40, 64, 2, 1088, False, "nonprefix"),
+                                                   (16, 128, 128, 2, 1088, True, None)])
+def test_auto_runs_fused_ln(device, b, s, d, h, f, causal, kind):
+    """What the automatic plan still gives to the fused-LN tiles: few tokens of a narrow model whose ffn_dim the
+    row chain does not take."""
+    from tttj_2026_amd import PLAN_AUTO, _lib
+    assert _lib.resolve_plan(b, s, d, h, f, PLAN_AUTO) == PLAN_FUSED_LN
+    cfg = TransformerConfig(b, s, d, h, f, 2, causal)
+    x16, _ = make_inputs(cfg, False, 47)
+    mask = _mask(kind, b, s, 48)
+    if mask is not None:
+        x16 = x16.masked_fill(~mask[..., None], 0)
+    gm = build_model(cfg, seed=49).half().to(device).eval()
+    opt = make_optimized_transformer(copy.deepcopy(gm))
+    fz = make_optimized_transformer(copy.deepcopy(gm), plan=PLAN_FUSED_LN)
+    xd, md = x16.to(device), None if mask is None else mask.to(device)
+    with torch.inference_mode():
+        y, yf = opt(xd, md), fz(xd, md)
+    res = O.check_tolerance(y, O.forward(O.params_fp32(gm), x16.float(), mask, h, causal), mask)
+    assert res["passed"], res
+    assert torch.equal(y, yf)
 
 
 def test_fused_ln_graph_replay(device):

@@ -211,7 +211,7 @@ def test_linear_rejects_bad_shapes(device):
                                    (4096, 32, 96), (64, 64, 8)])
 @pytest.mark.parametrize("masked", [False, True])
 def test_linear_small_shapes(device, m, n, k, mode, masked):
-    """N or K not a multiple of 64 (d_model 32, 96, ...): the vector-ALU kernel, same epilogues,
+    """N or K not a multiple of 64 (d_model 32, 96, ...): the ragged tiles, same epilogues,
     masked rows filled bitwise as on the MFMA path."""
     x = _rand((m, k), 110 + m, 1.0)
     w = _rand((n, k), 111 + n, 1.0 / math.sqrt(k))

@@ -70,3 +70,38 @@ def test_folded_layernorm_ragged(device, b, s, d, h, f, layers, scale, kind):
     res = O.check_tolerance(y1, O.forward(O.params_fp32(gm), x16.float(), mask, h, True), mask)
     assert res["passed"], res
     assert torch.equal(y1, y2)
+
+
+@pytest.mark.parametrize("kind", ["prefix", "scattered", "allvalid"])
+@pytest.mark.parametrize("b,s,d,h,f,causal", [
+    (8, 520, 72, 9, 144, False),     # head_dim 8, 64 x 64 tiles, partial column tiles of every part
+    (8, 300, 288, 9, 584, True),     # S % 8 != 0, ffn_dim off the 64 grid too
+    (5, 333, 480, 15, 968, False),   # odd S: V^T a value at a time
+    (16, 512, 480, 15, 960, True),   # 128 x 128 tiles
+])
+def test_packed_rows_ragged(device, b, s, d, h, f, causal, kind):
+    """The device's row count, the row map of the QKV epilogue and partial column tiles together: against the
+    oracle, and bit for bit against the forward that runs every token (the same tiles' arithmetic)."""
+    assert _lib.forward_packs_rows(b, s, d, h, f), "shape expected to run on packed rows"
+    cfg = TransformerConfig(b, s, d, h, f, 2, causal)
+    gm = _model(cfg, device, d)
+    x16, mask = _inputs(cfg, "none" if kind == "allvalid" else kind, s)
+    if mask is None:
+        mask = torch.ones(b, s, dtype=torch.bool)
+    opt = make_optimized_transformer(copy.deepcopy(gm))
+    xd, md = x16.to(device), mask.to(device)
+    with torch.inference_mode():
+        y1, y2 = opt(xd, md).clone(), opt(xd, md).clone()
+        _lib.check(_lib.load().tt_forward_packing_override(0), "packing override")
+        try:
+            y_pad = opt(xd, md).clone()
+        finally:
+            _lib.load().tt_forward_packing_override(-1)
+        y_none = opt(xd, None)
+    assert torch.equal(y1, y2) and torch.equal(y1, y_pad)
+    if kind == "allvalid":
+        assert torch.equal(y1, y_none)
+    idx = torch.arange(min(b, 6))  # sequences are independent
+    ref = O.forward(O.params_fp32(gm), x16[idx].float(), mask[idx], h, causal)
+    res = O.check_tolerance(y1.cpu()[idx], ref, mask[idx])
+    assert res["passed"], res

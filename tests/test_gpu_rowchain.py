@@ -41,7 +41,7 @@ def test_row_chain(device, b, s, d, h, f, layers, causal, mask_kind):
         mask[b // 2] = False  # a sequence without any valid token
     gm = model.half().to(device)
     y = {}
-    with torch.inference_mode():
+    with torch.inference_mode():  # the automatic plan and the explicit one, both of which run the row chain
         for plan in (None, PLAN_LAYERWISE):
             opt = make_optimized_transformer(gm) if plan is None else make_optimized_transformer(gm, plan=plan)
             md = None if mask is None else mask.to(device)
