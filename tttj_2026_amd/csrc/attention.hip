@@ -1,8 +1,9 @@
 // Flash-attention launches for head_dim 32, 64 and 128 (attention_kernel, one block per (b, h,
 // 128-query tile); the block itself is attention_block() in attention_block.hpp), the head_dim
 // dispatch (8 / 16: attention_small.hip, 256: attention_wide.hip) and the per-sequence mask
-// summary.  Built with the VGPR-form MFMA flag (accumulators in architectural VGPRs: 138-140 VGPRs
-// at head_dim 64, three waves per SIMD; 199-203 at 128, two).
+// summary.  Built with the VGPR-form MFMA flag (accumulators in architectural VGPRs: 146-148 VGPRs
+// at head_dim 64, 163 with two wave groups, three waves per SIMD; 199-203 at 128, two, and 256 with
+// four spilled with two wave groups).
 #include "attention_block.hpp"
 #include "kernels.hpp"
 

@@ -131,15 +131,19 @@ static bool packs_rows(bool fused_ln, bool fold, int64_t B, int64_t S, int64_t D
 // Whether the layer-wise and fused-LN plans run each layer as attention + row chain (rowchain.hip): narrow
 // models, where a 32-row block's share of the layer's weights streams from the L2 faster than five to seven
 // launches.  Measured on MI355X, whole forwards, launches per op -> row chain: D 128, F 128, 4 layers, S 128: B 1
-// 93 -> 51 us (fused-LN tiles), B 64 144 -> 67, B 10000 7576 -> 4970; D 128, F 512, 32 x 1024 tokens, 2 layers
-// 200 -> 122; D 192, F 768 the same 250 -> 203; D 160, F 640, 1600 tokens, one layer 40 -> 29.  At D 256 every block
-// streams four times the bytes of D 128 and the GEMM tiles win (4 x 128 tokens, F 1024: 60 -> 123 us; 32 x 512: 192
-// -> 252, with a first form of the kernel).
+// 93 -> 51 us (fused-LN tiles), B 64 144 -> 65, B 10000 7576 -> 4970; D 128, F 512, 32 x 1024 tokens, 2 layers
+// 200 -> 122; D 192, F 768 the same 250 -> 203; D 160, F 640, 1600 tokens, one layer 40 -> 26.  D 256 stays with the
+// GEMM tiles: every block streams four times the bytes of D 128, and the row chain loses with few tokens and with
+// many (two layers: 128 tokens, F 256 40.2 -> 46.3 us, 512 tokens, F 1024 50.4 -> 64.3, 65536 tokens, F 256 444 ->
+// 486), though not between (4096 tokens, F 256 78.5 -> 57.4; 16384, F 1024 191 -> 157).  Padded batches of more than
+// 2^20 tokens pack their rows, which callers can ask for (tt_forward_packs_rows); the row chain would be as fast or
+// faster there too (four layers, 10000 x 128 tokens, launches on packed rows -> row chain: D 128 = F 6216 -> 5226
+// us, D 192 = F 10469 -> 10464).
 static bool chains_rows(bool masked, int64_t B, int64_t S, int64_t D, int64_t H, int64_t F) {
   const int64_t T = B * S, Sp = (S + 63) / 64 * 64;
   if (chain_fragment_halfs(D, F) == 0) return false;
   if (T * D >= (1LL << 31) || B * D * Sp >= (1LL << 31)) return false;
-  return !masked || T <= (1LL << 20);  // larger padded batches pack their rows
+  return !masked || T <= (1LL << 20);
 }
 
 static int check_model_shape(int B, int S, int D, int H, int F, int L) {
@@ -206,8 +210,11 @@ static constexpr int kMegaMaxDModel = 512;  // the megakernel keeps a LayerNorm'
 // gains up to 2048 tokens (the reference's cases 2-4: 94 / 92 / 102 us fused against 101 / 97 /
 // 115 layer-wise) and loses from 8192 (case 1: 161 against 147 us); at d_model 256 the layer-wise
 // plan with narrow GEMM tiles is as fast or faster (C1 68 / 68 us, C2 106 against 118 us).  Both
-// plans take the row chain first where it applies (chains_rows), which leaves the tiles ffn_dim
-// above 1024 and explicit plans above d_model 192.
+// plans take the row chain first where it applies (chains_rows), those cases among them, which leaves
+// the tiles ffn_dim above 1024 and explicit plans above d_model 192.  There the narrow tiles have caught
+// up since (two layers, fused against layer-wise: d_model 64, F 1280, 64 / 1024 / 2048 tokens 40.1 / 52.5
+// / 62.7 against 38.9 / 53.0 / 61.4 us; d_model 128 44.3 / 60.5 / 80.1 against 40.1 / 58.2 / 73.0); the
+// automatic plan's choice is part of the interface and stays.
 static constexpr int64_t kFusedLnMaxTokens = 2048;
 static constexpr int kFusedLnMaxDModel = 128;
 

@@ -111,10 +111,10 @@ static bool is_ragged(int n, int k) { return k % kBK != 0 || n % 64 != 0; }
 
 // Tile choice for ragged widths (no width of these models divides a tile, so the partial last tile of
 // each row counts as whole): 128 x 128 once its tiles reach every CU (measured on MI355X against
-// 64 x 64: 6000 x 1000 x 1000 35.8 -> 29.0 us, 4096 x 1000 x 1000 24.3 -> 18.6; at 10000 x 480 x 480
-// 15.7 -> 16.8, the worst of ten shapes), 32 x 32 narrow tiles where 64 x 64 would fill at most half the
-// CUs (the rule of the aligned widths), else 64 x 64.  Against the vector-ALU kernel these replaced:
-// 1600 x 480 x 160 (QKV) 58 -> 5 us, 1600 x 640 x 160 91 -> 6 us.
+// 64 x 64: 6000 x 1000 x 1000 35.8 -> 29.0 us, 4096 x 1000 x 1000 24.3 -> 18.6; one of ten shapes loses,
+// 10000 x 480 x 480 15.7 -> 16.8), 32 x 32 narrow tiles where 64 x 64 would fill at most half the CUs (the
+// rule of the aligned widths), else 64 x 64.  Against the vector-ALU kernel these replaced: 1600 x 480 x 160
+// (QKV) 58 -> 5 us, 1600 x 640 x 160 91 -> 6 us.
 // Rows of 2^22 values and more stay on the narrow tiles, which address each row by a pointer: the others mark
 // loads past K by a buffer offset just below 2^31, which has to lie past the tile's 128 rows.
 static RaggedTile pick_ragged(int m, int n, int k, int mode, int cus) {

@@ -108,7 +108,7 @@ struct AttnArgs;
 // head_dim 256: the MFMA flash block with accumulators in AGPRs (attention_wide.hip).
 int launch_attention_wide(const AttnArgs& args, const int32_t* info, int head_dim, int causal,
                           hipStream_t stream);
-// head_dim 8 / 16: 16-wide MFMA tiles, probabilities in fp32 precision (attention_small.hip).
+// head_dim 8 / 16: 16-wide MFMA tiles, probabilities of 22 bits (attention_small.hip).
 int launch_attention_small(const AttnArgs& args, const int32_t* info, int head_dim, int causal,
                            hipStream_t stream);
 

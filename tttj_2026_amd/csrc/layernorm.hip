@@ -1,8 +1,8 @@
 // Row LayerNorm for the pre-LN block stack (norm1 / norm2 / final_norm) on gfx950.
 //
-// G lanes own one row of D fp16 values (D <= 8192): a whole wave for D > 256, 32, 16 or 8 lanes for narrower
-// rows, so that no lane is without a 16-byte chunk (one row per wave left 48 of 64 lanes idle at D = 128:
-// 65536 x 128 14.0 -> 6.0 us on MI355X, 30000 x 256 8.0 -> 5.6).  Every lane loads its chunks once into
+// G lanes own one row of D fp16 values (D <= 8192): a whole wave for D > 256, else the smallest of 8, 16 and 32
+// lanes that has one for each 16-byte chunk (one row per wave left 48 of 64 lanes idle at D = 128: 65536 x 128
+// 14.0 -> 6.0 us on MI355X, 30000 x 256 8.0 -> 5.6).  Every lane loads its chunks once into
 // registers, the lanes reduce the mean, then the centred second moment (two-pass, fp32), and write
 // (x - mean) * rsqrt(var + eps) * gamma + beta as fp16.  Rows whose mask byte is zero are written as +0.0
 // (the final_norm + masked_fill of torch_transformer_benchmark.py:169-171).

@@ -1,4 +1,4 @@
-// Row-chain kernel for narrow models (d_model 32 ... 256): everything of a layer between two attentions in
+// Row-chain kernel for narrow models (d_model 32 ... 192): everything of a layer between two attentions in
 // one launch.
 //
 // For R = 16 RT rows (tokens) of the residual stream one 512-thread block runs, with every intermediate in
@@ -19,10 +19,12 @@
 // Weights are read from their fragment-order copies (launch_pack_fragments): a wave's load is 1 KiB contiguous.
 // Read from the row-major matrices, 16 rows x 64 bytes per instruction, a load holds the address unit for 64
 // cycles: 196 KB (all weights of D = F = 128) take 12800 cycles instead of 4300 per CU, and a 32-row tile at
-// D = F = 128 took 21800 cycles, with its Q / K / V^T stored from the accumulators, instead of 15800.  Where a block walks several tiles (KEEP) it reads them once.
+// D = F = 128 took 21800 cycles, with its Q / K / V^T stored from the accumulators, instead of 15800.  Where a
+// block walks several tiles (KEEP) it reads them once.
 // Cycles of one 32-row tile at D = F = 128 (14600): rows and weights arriving 3700, out_proj 2400, LN2 1200, FFN
-// 2600, ffn_out and its epilogue 900, LN1 1100, QKV 2300, stores 500.  64-row tiles (more rows than 32 per
-// CU) are bound by the vector work of the epilogues (GELU, conversions, LayerNorm) and the fragment reads.
+// 2600, ffn_out and its epilogue 900, LN1 1100, QKV 2300, stores 500.  64-row tiles are bound by the vector
+// work of the epilogues (GELU, conversions, LayerNorm) and the fragment reads; with the weights kept they spill
+// registers (15 at D 96, 51 at D 128).
 // For the V part of the QKV projection the operands change places, so that a lane ends with 4 consecutive
 // tokens of one feature: pieces of V^T rows without a transposing pass.
 #include "common.hpp"
@@ -510,6 +512,11 @@ static int run_chain_mid(const ChainArgs& a, bool mid, hipStream_t stream) {
   return mid ? run_chain<D, RT, true, KEEP>(a, stream) : run_chain<D, RT, false, KEEP>(a, stream);
 }
 
+// 64-row tiles beyond 32 rows per CU.  Measured on MI355X, forwards of two layers, 32-row -> 64-row tiles: 1024 to
+// 7680 tokens 7% (D 32) to 44% (D 128) slower; 16384 tokens D 32 31.7 -> 27.2 us, D 64 37.2 -> 29.8, D 96 51.0 ->
+// 50.0, D 128 with F 512 68.3 -> 67.0; 65536 tokens D 32 81.3 -> 64.9, D 64 97.4 -> 78.6 (F 256 92.1 -> 95.6),
+// D 96 125.8 -> 118.7, D 128 with F 512 200.9 -> 186.4.  The line is wrong for the spilling form at D = F = 128:
+// 16384 tokens 54.6 -> 57.8 us, 65536 125.8 -> 141.1.
 template <int D>
 static int run_chain_d(const ChainArgs& a, bool mid, hipStream_t stream) {
   const bool many = a.T > 32 * device_cus();
