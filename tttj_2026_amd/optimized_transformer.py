@@ -314,10 +314,11 @@ class OptimizedTransformer(nn.Module):
             raise ValueError(f"x must be [B, S, {cfg.d_model}], got {tuple(x.shape)}")
         if x.dtype != torch.float16 or x.device.type != "cuda":
             raise ValueError("x must be a CUDA float16 tensor")
-        if self.packed_weights.device != x.device or self.packed_weights.dtype != torch.float16:
+        packed = self.packed_weights  # (a buffer of a module: each access costs a lookup)
+        if packed.device != x.device or packed.dtype != torch.float16:
             raise ValueError("packed weights and input must be fp16 on the same device")
-        if self.packed_weights.numel() < self._weight_elems:  # the library is given no size
-            raise ValueError(f"packed weights of {self.packed_weights.numel()} elements, the layout has "
+        if packed.numel() < self._weight_elems:  # the library is given no size
+            raise ValueError(f"packed weights of {packed.numel()} elements, the layout has "
                              f"{self._weight_elems} (packed by another version?)")
         batch, seq, _ = x.shape
         x = x.contiguous()
@@ -340,7 +341,7 @@ class OptimizedTransformer(nn.Module):
         self.last_mask = valid_token_mask
         stream = torch.cuda.current_stream(x.device).cuda_stream
         rc = self._lib.tt_transformer_fwd(
-            self.packed_weights.data_ptr(), x.data_ptr(), mask_ptr, y.data_ptr(), ws.data_ptr(),
+            packed.data_ptr(), x.data_ptr(), mask_ptr, y.data_ptr(), ws.data_ptr(),
             ws.numel(), batch, seq, cfg.d_model, cfg.num_heads, cfg.ffn_dim, cfg.num_layers,
             int(bool(cfg.causal)), plan, stream)
         _lib.check(rc, "tt_transformer_fwd")
